@@ -647,14 +647,9 @@ torch::Tensor gemv_f16(torch::Tensor weight, torch::Tensor x) {
     auto out_shape = xf.sizes().vec();
     out_shape.back() = out_dim;
     torch::Tensor out = torch::empty(out_shape, w.options());
-    const int dev = w.get_device();
-    for (int64_t r0 = 0; r0 < rows; r0 += 8) {
-        const int64_t nb = std::min<int64_t>(8, rows - r0);
-        check(gdsllm_gemv_f16(w.data_ptr(), static_cast<const at::Half*>(xf.data_ptr()) + r0 * in_dim,
-                              static_cast<at::Half*>(out.data_ptr()) + r0 * out_dim, out_dim, in_dim, nb, in_dim,
-                              out_dim, OnDevice(dev).stream()),
-              where);
-    }
+    check(gdsllm_gemv_f16_tokens(w.data_ptr(), xf.data_ptr(), out.data_ptr(), out_dim, in_dim, rows, in_dim, out_dim,
+                                 OnDevice(w.get_device()).stream()),
+          where);
     return out;
 }
 

@@ -91,13 +91,18 @@ __device__ __forceinline__ void f16_row_parts(const uint16_t* __restrict__ wr, c
     }
 }
 
-// Rows blockIdx.x, += gridDim.x: y[b][r] = fp16(((p0 + p1) + p2) + p3).
+// Rows blockIdx.x, += gridDim.x of x rows nb*blockIdx.y .. +nb-1 (fewer past
+// T): y[b][r] = fp16(((p0 + p1) + p2) + p3).
 template <int NJ>
 __global__ __launch_bounds__(kF16Waves * 64) void gemv_f16(const uint16_t* __restrict__ W,
                                                            const uint16_t* __restrict__ X, uint16_t* __restrict__ Y,
-                                                           int M, int K, int nb, int64_t ldx, int64_t ldy) {
+                                                           int M, int K, int nb, int64_t T, int64_t ldx, int64_t ldy) {
     __shared__ float part[4][kMaxBatch];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t t0 = static_cast<int64_t>(blockIdx.y) * nb;
+    X += t0 * ldx;
+    Y += t0 * ldy;
+    nb = static_cast<int>(min(static_cast<int64_t>(nb), T - t0));
     for (int r = blockIdx.x; r < M; r += gridDim.x) {
         f16_row_parts<NJ>(W + static_cast<int64_t>(r) * K, X, K, nb, ldx, wave, lane, part);
         __syncthreads();
@@ -112,7 +117,11 @@ __global__ __launch_bounds__(kF16Waves * 64) void gemv_f16(const uint16_t* __res
 __global__ __launch_bounds__(kF16Waves * 64) void gemv_f16_scalar(const uint16_t* __restrict__ W,
                                                                   const uint16_t* __restrict__ X,
                                                                   uint16_t* __restrict__ Y, int M, int K, int nb,
-                                                                  int64_t ldx, int64_t ldy) {
+                                                                  int64_t T, int64_t ldx, int64_t ldy) {
+    const int64_t t0 = static_cast<int64_t>(blockIdx.y) * nb;
+    X += t0 * ldx;
+    Y += t0 * ldy;
+    nb = static_cast<int>(min(static_cast<int64_t>(nb), T - t0));
     const int lane = threadIdx.x & 63;
     const int wpb = static_cast<int>(blockDim.x) >> 6;
     const int nwaves = static_cast<int>(gridDim.x) * wpb;
@@ -187,45 +196,89 @@ __global__ __launch_bounds__(256) void moe_combine(const uint16_t* __restrict__ 
 
 using namespace gdsllm;
 
+namespace {
+// y[t][r] for T rows of x, nb of them per workgroup (grid.y).
+int gemv_f16_run(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim, int64_t T, int nb,
+                 int64_t ldx, int64_t ldy, void* stream) {
+    const int M = static_cast<int>(out_dim), K = static_cast<int>(in_dim);
+    const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(x) % 16 == 0 && (T == 1 || ldx % 8 == 0);
+    const auto* w = static_cast<const uint16_t*>(weight);
+    const hipStream_t st = as_stream(stream);
+    const int64_t most = int64_t(65535) * nb;  // x rows of one launch: grid.y is 16 bits
+    for (int64_t t = 0; t < T; t += most) {
+        const int64_t n = std::min(most, T - t);
+        const auto* xp = static_cast<const uint16_t*>(x) + t * ldx;
+        auto* yp = static_cast<uint16_t*>(y) + t * ldy;
+        const unsigned gy = static_cast<unsigned>((n + nb - 1) / nb);
+        if (vec) {
+            // a 4-wave workgroup per row (one row each while the grid fits)
+            const int grid = std::min(M, 16 * cu_count());
+            const int nj = ((K + 511) / 512 + 3) / 4;
+            auto launch = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(grid, gy), dim3(kF16Waves * 64), 0, st, w, xp, yp, M, K, nb, n, ldx, ldy);
+            };
+            if (nj <= 1) launch(gemv_f16<1>);
+            else if (nj <= 2) launch(gemv_f16<2>);
+            else if (nj <= 4) launch(gemv_f16<4>);
+            else launch(gemv_f16<0>);
+        } else {
+            const int grid = std::min((M + kF16Waves - 1) / kF16Waves, 8 * cu_count());
+            hipLaunchKernelGGL(gemv_f16_scalar, dim3(grid, gy), dim3(kF16Waves * 64), 0, st, w, xp, yp, M, K, nb, n,
+                               ldx, ldy);
+        }
+        if (int rc = check_hip(hipGetLastError(), "gemv_f16 launch")) return rc;
+    }
+    return ok();
+}
+
+int check_gemv_f16(const std::string& n, const void* weight, const void* x, const void* y, int64_t out_dim,
+                   int64_t in_dim, int64_t T, int64_t ldx, int64_t ldy, bool& empty) {
+    empty = false;
+    if (out_dim > (int64_t(1) << 30) || in_dim > (int64_t(1) << 24))
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": dimension too large");
+    if (out_dim == 0 || in_dim == 0 || T == 0) {
+        empty = true;
+        return GDSLLM_OK;
+    }
+    if (!weight || !x || !y) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": null pointer");
+    if (T > 1 && (ldx < in_dim || ldy < out_dim))
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": ldx/ldy smaller than the row length");
+    if (reinterpret_cast<uintptr_t>(weight) % 2 || reinterpret_cast<uintptr_t>(x) % 2 ||
+        reinterpret_cast<uintptr_t>(y) % 2)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": weight, x and y must be 2-byte aligned");
+    return GDSLLM_OK;
+}
+}  // namespace
+
 extern "C" int gdsllm_gemv_f16(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
                                int64_t batch, int64_t ldx, int64_t ldy, void* stream) {
     const std::string n = "gemv_f16";
     if (out_dim < 0 || in_dim < 0) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": negative dimension");
     if (batch < 1 || batch > kMaxBatch)
         return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": batch must be in [1, 8], got " + std::to_string(batch));
-    if (out_dim > (int64_t(1) << 30) || in_dim > (int64_t(1) << 24))
-        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": dimension too large");
-    if (out_dim == 0 || in_dim == 0) return ok();
-    if (!weight || !x || !y) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": null pointer");
-    if (batch > 1 && (ldx < in_dim || ldy < out_dim))
-        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": ldx/ldy smaller than the row length");
-    if (reinterpret_cast<uintptr_t>(weight) % 2 || reinterpret_cast<uintptr_t>(x) % 2 ||
-        reinterpret_cast<uintptr_t>(y) % 2)
-        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": weight, x and y must be 2-byte aligned");
-    const int M = static_cast<int>(out_dim), K = static_cast<int>(in_dim), B = static_cast<int>(batch);
-    const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(weight) % 16 == 0 &&
-                     reinterpret_cast<uintptr_t>(x) % 16 == 0 && (B == 1 || ldx % 8 == 0);
-    const auto* w = static_cast<const uint16_t*>(weight);
-    const auto* xp = static_cast<const uint16_t*>(x);
-    auto* yp = static_cast<uint16_t*>(y);
-    const hipStream_t st = as_stream(stream);
-    if (vec) {
-        // a 4-wave workgroup per row (one row each while the grid fits)
-        const int grid = std::min(M, 16 * cu_count());
-        const int nj = ((K + 511) / 512 + 3) / 4;
-        auto launch = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(grid), dim3(kF16Waves * 64), 0, st, w, xp, yp, M, K, B, ldx, ldy);
-        };
-        if (nj <= 1) launch(gemv_f16<1>);
-        else if (nj <= 2) launch(gemv_f16<2>);
-        else if (nj <= 4) launch(gemv_f16<4>);
-        else launch(gemv_f16<0>);
-    } else {
-        const int grid = std::min((M + kF16Waves - 1) / kF16Waves, 8 * cu_count());
-        hipLaunchKernelGGL(gemv_f16_scalar, dim3(grid), dim3(kF16Waves * 64), 0, st, w, xp, yp, M, K, B, ldx, ldy);
-    }
-    if (int rc = check_hip(hipGetLastError(), "gemv_f16 launch")) return rc;
-    return ok();
+    bool empty;
+    if (int rc = check_gemv_f16(n, weight, x, y, out_dim, in_dim, batch, ldx, ldy, empty)) return rc;
+    if (empty) return ok();
+    return gemv_f16_run(weight, x, y, out_dim, in_dim, batch, static_cast<int>(batch), ldx, ldy, stream);
+}
+
+extern "C" int gdsllm_gemv_f16_tokens(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                      int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+    const std::string n = "gemv_f16_tokens";
+    if (out_dim < 0 || in_dim < 0 || tokens < 0)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": negative dimension");
+    bool empty;
+    if (int rc = check_gemv_f16(n, weight, x, y, out_dim, in_dim, tokens, ldx, ldy, empty)) return rc;
+    if (empty) return ok();
+    // Up to 8 x rows share a workgroup's weight row; fewer where that would
+    // leave less than two workgroups per CU.  Each output is one wave-ordered
+    // sum over its own rows of W and x, so nb does not change its bits.  The
+    // 1 x 4096 shared-expert gate over 512 tokens: 64 launches of 8 tokens
+    // took 478 us (kernel trace sum), this one launch, one token per workgroup, 5.3.
+    const int64_t per = out_dim * std::min<int64_t>(tokens, int64_t(1) << 20) / (2 * static_cast<int64_t>(cu_count()));
+    const int nb = static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(kMaxBatch, per)));
+    return gemv_f16_run(weight, x, y, out_dim, in_dim, tokens, nb, ldx, ldy, stream);
 }
 
 extern "C" int gdsllm_moe_route_topk(const void* logits, int64_t num_experts, int64_t n_tok, int64_t ld_logits,

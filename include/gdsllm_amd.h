@@ -273,6 +273,12 @@ int gdsllm_moe_step_routed_affine_q4(const void* router_weight, const gdsllm_aff
 int gdsllm_gemv_f16(const void* weight, const void* x, void* y,
                     int64_t out_dim, int64_t in_dim, int64_t batch,
                     int64_t ldx, int64_t ldy, void* stream);
+/* The same for any number of x rows in one launch (per 65535 workgroups along
+ * the rows): a prefill chunk's shared-expert gate.  Each output has the bits
+ * gdsllm_gemv_f16 gives it.                                                 */
+int gdsllm_gemv_f16_tokens(const void* weight, const void* x, void* y,
+                           int64_t out_dim, int64_t in_dim, int64_t tokens,
+                           int64_t ldx, int64_t ldy, void* stream);
 
 /* Per token t < n_tok, from fp16 logits at logits + t*ld_logits: the top_k
  * largest in descending order into idx[t*top_k ...] (int32) and

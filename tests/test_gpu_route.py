@@ -30,6 +30,25 @@ def test_gemv_f16(gpu, M, K, B, w_off):
     assert_gemv_close(to_np(y), to_np(w), to_np(x), f"gemv_f16 {M}x{K} b{B} off{w_off}")
 
 
+@pytest.mark.parametrize("M,K,T", [(1, 4096, 512), (1, 4096, 9), (3, 2048, 1025), (513, 512, 17), (1, 100, 33),
+                                   (2, 12288, 65), (1, 8, 600000)])
+def test_gemv_f16_tokens(gpu, M, K, T):
+    """Any number of x rows in one call: the bits of the 8-row launches (the
+    last case spans more workgroups along the rows than one grid dimension holds)."""
+    g = gen(6050 + M + K + T)
+    w = (torch.randn(M, K, generator=g, device=g.device) * 0.05).to(torch.float16).to(gpu)
+    x = torch.randn(T, K + 8, generator=gen(6051 + K), device=g.device).to(torch.float16).to(gpu)
+    y = torch.full((T + 1, M + 1), 7.0, dtype=torch.float16, device=gpu)
+    check(capi().gdsllm_gemv_f16_tokens(ptr(w), ptr(x), ptr(y), M, K, T, K + 8, M + 1, stream()))
+    sample = range(0, T, 8) if T < 2000 else [0, 8, 65528, 65536, 524280, 524288, T - 8]
+    for t in sample:
+        n = min(8, T - t)
+        want = torch.empty(n, M, dtype=torch.float16, device=gpu)
+        check(capi().gdsllm_gemv_f16(ptr(w), ptr(x[t]), ptr(want), M, K, n, K + 8, M, stream()))
+        assert torch.equal(y[t:t + n, :M].view(torch.int16), want.view(torch.int16))
+    assert bool((y[T] == 7).all()) and bool((y[:, M] == 7).all())
+
+
 def _ulp_close(got: np.ndarray, want: np.ndarray, what: str, min_exact: float = 0.95):
     g, w = got.astype(np.float16), want.astype(np.float16)
     same = (g.view(np.uint16) == w.view(np.uint16)) | (np.isnan(g) & np.isnan(w))
