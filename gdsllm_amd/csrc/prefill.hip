@@ -62,7 +62,7 @@
 
 #include <algorithm>
 
-#include "common.h"
+#include "moe_stream.h"
 
 namespace gdsllm {
 namespace {
@@ -108,7 +108,8 @@ struct Fmt {
 // workgroups share a CU and one's pipeline fill and epilogue overlap the
 // other's stream: each tile job is short (one expert's ~10 tokens), and with
 // 6 + 5 slots (139 KiB, one workgroup per CU) the 512-token chunk over the
-// 512-expert pool took 1560 us, with 4 + 2 slots 1178-1227 us.
+// 512-expert pool took 1560 us, with 4 + 2 slots 1178-1227 us (chunks with few
+// tokens per expert, as that one, now run in moe_stream.hip).
 template <WF F, int BT, int BM = kBM>
 struct Ring {
     static constexpr int kXSlot = BT * 256;
@@ -878,6 +879,17 @@ __global__ __launch_bounds__(256) void moe_prefill_combine(const uint16_t* __res
 }
 
 constexpr int kMoeBT = 32;
+// Mean tokens per expert up to which the chunk runs as weight streams
+// (moe_stream.hip) instead of the split-K tiles below: a stream pass serves 16
+// tokens of an expert, the tiles 32 for one dequantization.  Measured, us per
+// chunk with the shared expert, tiles against streams: 512 experts of 1024 x
+// 4096 at a mean of 1 / 5 / 10 / 14 / 18 tokens 701 / 1055 / 1107 / 1154 / 1187
+// against 510 / 729 / 815 / 1012 / 1278; 256 of 768 x 3072 at 5 / 10 / 14 / 18
+// 349 / 372 / 387 / 400 against 254 / 342 / 379 / 449; 128 of 512 x 2048 at 5 /
+// 10 / 14 / 18 137 / 143 / 141 / 150 against 108 / 142 / 141 / 162; 64 of 1024
+// x 4096, whose few jobs leave the longest expert as the tail, at 5 / 10 / 14
+// 197 / 199 / 203 against 145 / 205 / 207.
+inline int64_t stream_tokens(int64_t experts) { return experts >= 128 ? 10 : 8; }
 
 struct PrefillLayout {
     size_t tok, pos, tiles, ntiles, h, d, total;
@@ -920,6 +932,48 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
                        static_cast<int>(E), kMoeBT, tok, pos, tiles, ntiles);
     if (int rc = check_hip(hipGetLastError(), "moe_sort launch")) return rc;
     const int64_t max_tiles = n / kMoeBT + std::min<int64_t>(E, n);
+    auto combine = [&]() {
+        const int64_t threads = T * (H / 8);
+        hipLaunchKernelGGL(moe_prefill_combine, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
+                           dbuf, pos, static_cast<const uint16_t*>(rw), static_cast<int>(k), static_cast<int>(H),
+                           static_cast<int>(T), static_cast<uint16_t*>(y), ldy);
+        return check_hip(hipGetLastError(), "moe_prefill_combine launch");
+    };
+    if (n <= stream_tokens(E) * E && moe_stream_fits(Fd, H) && moe_stream_fits(H, Fd)) {
+        auto pool = [](const gdsllm_affine_experts& p, const gdsllm_affine_experts& p2) {
+            MoeStreamArgs a{};
+            a.w = static_cast<const uint8_t*>(p.weight);
+            a.s = static_cast<const uint8_t*>(p.scales);
+            a.b = static_cast<const uint8_t*>(p.biases);
+            a.w2 = static_cast<const uint8_t*>(p2.weight);
+            a.s2 = static_cast<const uint8_t*>(p2.scales);
+            a.b2 = static_cast<const uint8_t*>(p2.biases);
+            a.estride_w = p.weight_stride;
+            a.estride_s = p.scale_stride;
+            a.estride_b = p.bias_stride;
+            a.M = static_cast<int>(p.out_dim);
+            a.K = static_cast<int>(p.in_dim);
+            return a;
+        };
+        MoeStreamArgs a = pool(g, u);
+        a.x = static_cast<const uint16_t*>(x);
+        a.ldx = ldx;
+        a.tok = tok;
+        a.y = hbuf;
+        a.ldy = Fd;
+        a.tiles = tiles;
+        a.ntiles = ntiles;
+        if (int rc = moe_stream(a, static_cast<int>(g.group_size), true, max_tiles, stream)) return rc;
+        MoeStreamArgs b = pool(d, d);
+        b.x = hbuf;  // h rows by position
+        b.ldx = Fd;
+        b.y = dbuf;
+        b.ldy = H;
+        b.tiles = tiles;
+        b.ntiles = ntiles;
+        if (int rc = moe_stream(b, static_cast<int>(g.group_size), false, max_tiles, stream)) return rc;
+        return combine();
+    }
 
     GemmArgs a{};
     a.w = static_cast<const uint8_t*>(g.weight);
@@ -966,12 +1020,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     b.ntiles = ntiles;
     b.tok = nullptr;
     if (int rc = launch_sk<F, kMoeBT, kGather>(b, static_cast<unsigned>(max_tiles * b.mtiles), stream)) return rc;
-
-    const int64_t threads = T * (H / 8);
-    hipLaunchKernelGGL(moe_prefill_combine, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
-                       dbuf, pos, static_cast<const uint16_t*>(rw), static_cast<int>(k), static_cast<int>(H),
-                       static_cast<int>(T), static_cast<uint16_t*>(y), ldy);
-    return check_hip(hipGetLastError(), "moe_prefill_combine launch");
+    return combine();
 }
 
 }  // namespace

@@ -239,6 +239,33 @@ def test_moe_prefill(gpu, E, H, F, g, k, T):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
+# (E, H, F, g, k, T) with few tokens per expert, the streamed form: K of 256 and
+# 768 (half-size units), 512 and 1536 (scales of one unit a load), 1024 and 2048
+# (two and four), rows past a job's range (H = 1280), every group size
+STREAM_CASES = [(40, 1024, 512, 64, 4, 30), (40, 768, 256, 64, 2, 40), (24, 2048, 1024, 128, 3, 20),
+                (24, 1536, 512, 32, 3, 20), (24, 1280, 768, 128, 2, 30), (130, 512, 256, 32, 4, 200),
+                (24, 2048, 256, 32, 2, 9)]
+
+
+@pytest.mark.parametrize("E,H,F,g,k,T", STREAM_CASES,
+                         ids=[f"E{e}_H{h}_F{f}_g{g}_k{k}_T{t}" for e, h, f, g, k, t in STREAM_CASES])
+def test_moe_prefill_few_tokens_per_expert(gpu, E, H, F, g, k, T):
+    """Every token also picks expert 1 in its first slot: one expert with T
+    tokens (tiles of 32 and a rest, 16 tokens a pass) beside ones with few or
+    none."""
+    gg = gen(5900 + E + T)
+    pools = [syn.affine_q4_weights(s, g, gg) for s in ([E, F, H], [E, F, H], [E, H, F])]
+    x = syn.activations(T, H, gen(5901 + T))
+    rest = [np.random.default_rng(5902 + t).choice(np.arange(2, E), k - 1, replace=False) for t in range(T)]
+    idx = np.stack([np.concatenate([[1], r]) for r in rest]).astype(np.int32)
+    wts = torch.softmax(torch.randn(T, k, generator=gen(5903)), -1).to(torch.float16)
+    dev = [tuple(t.to(gpu) for t in p) for p in pools]
+    y, tok, pos, tiles, hbuf, dbuf = moe_prefill(*dev, x.to(gpu), torch.from_numpy(idx).to(gpu), wts.to(gpu), g, T, k)
+    check_sort(idx, tok, pos, tiles, E)
+    check_moe_prefill(y, tok, pos, hbuf, dbuf, *pools, x, idx, to_np(wts), g, E,
+                      sample=sorted(set(range(0, T, 7)) | {15 % T, 16 % T, T - 1}))
+
+
 def test_moe_prefill_out_of_range_experts(gpu):
     E, H, F, g, k, T = 6, 512, 256, 64, 3, 11
     gg = gen(5700)
