@@ -504,6 +504,14 @@ std::optional<torch::Tensor> moe_step_affine_q4(torch::Tensor x, std::vector<Aff
     return out;
 }
 
+// The partial-sum workspace of a prefill GEMM that splits K, from torch's
+// allocator on the current stream (undefined where the library does not split).
+torch::Tensor gemm_workspace(int64_t out_dim, int64_t in_dim, int64_t tokens, int dev) {
+    const auto bytes = static_cast<int64_t>(gdsllm_dequant_gemm_workspace_size(out_dim, in_dim, tokens));
+    if (bytes == 0) return {};
+    return torch::empty({bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, dev));
+}
+
 // Prefill: x [..., in_dim] fp16 -> [..., out_dim] fp16 on the MFMA dequant-GEMM
 // (Q4_0 or Q8_0).  None when the library cannot serve the shape or alignment
 // (the caller then takes the reference's dequant -> F.linear route).
@@ -525,9 +533,10 @@ std::optional<torch::Tensor> fused_dequant_gemm(const Handle& h, torch::Tensor x
     auto out_shape = xf.sizes().vec();
     out_shape.back() = out_dim;
     torch::Tensor out = torch::empty(out_shape, fp16_on(h->device_id()));
-    const int rc = (q4 ? gdsllm_dequant_gemm_q4_0 : gdsllm_dequant_gemm_q8_0)(
+    torch::Tensor ws = gemm_workspace(out_dim, in_dim, tokens, h->device_id());
+    const int rc = (q4 ? gdsllm_dequant_gemm_q4_0_ws : gdsllm_dequant_gemm_q8_0_ws)(
         at_offset(h, offset), xf.data_ptr(), out.data_ptr(), out_dim, in_dim, tokens, in_dim, out_dim,
-        OnDevice(h->device_id()).stream());
+        ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, OnDevice(h->device_id()).stream());
     if (rc == GDSLLM_ERR_UNSUPPORTED) return std::nullopt;
     check(rc, where);
     return out;
@@ -587,8 +596,11 @@ std::optional<torch::Tensor> fused_affine_q4_gemm(const Handle& h, torch::Tensor
     auto out_shape = xf.sizes().vec();
     out_shape.back() = out_dim;
     torch::Tensor out = torch::empty(out_shape, fp16_on(h->device_id()));
-    const int rc = gdsllm_dequant_gemm_affine_q4(p.w, p.s, p.b, xf.data_ptr(), out.data_ptr(), out_dim, in_dim,
-                                                 group_size, tokens, in_dim, out_dim, OnDevice(h->device_id()).stream());
+    torch::Tensor ws = gemm_workspace(out_dim, in_dim, tokens, h->device_id());
+    const int rc = gdsllm_dequant_gemm_affine_q4_ws(p.w, p.s, p.b, xf.data_ptr(), out.data_ptr(), out_dim, in_dim,
+                                                    group_size, tokens, in_dim, out_dim,
+                                                    ws.defined() ? ws.data_ptr() : nullptr,
+                                                    ws.defined() ? ws.numel() : 0, OnDevice(h->device_id()).stream());
     if (rc == GDSLLM_ERR_UNSUPPORTED) return std::nullopt;
     check(rc, where);
     return out;

@@ -6,7 +6,7 @@
 // (runtime/llama.py:160-166 for GGUF Q4_0 / Q8_0, runtime/qwen_moe.py:72-73
 // for affine-Q4), fused so the fp16 weight matrix never goes back to HBM.
 //
-// One split-K workgroup kernel serves three weight formats and three modes.
+// One split-K workgroup kernel serves three weight formats and five modes.
 //
 // Workgroup: 128 weight rows x BT tokens (BT = 64 or 32), 8 waves (two per
 // SIMD).  A stage is 128 values of k (four 32-value blocks); wave w takes
@@ -54,6 +54,9 @@
 //             0..BM/2-1 from the gate matrix and BM/2..BM-1 from the up matrix
 //             at the same BM/2 output rows, h written instead of g and u (the
 //             prefill form of the decode gate_up_silu, runtime/llama.py:253-256).
+//  * kDenseSplit  kDense over one of several parts of K, with fp32 partial sums
+//             stored instead of Y (split_sum adds them in part order): for
+//             launches whose tiles leave most compute units idle.
 //  * kDualSilu  kGather with rows 0..63 of the workgroup taken from the gate
 //             pool and rows 64..127 from the up pool at the same 64 output
 //             rows; the epilogue writes h = fp16(fp16(silu(g)) * u) with
@@ -68,7 +71,7 @@ namespace gdsllm {
 namespace {
 
 enum class WF { Q4_0, Q8_0, AFF32, AFF64, AFF128 };
-enum Mode { kDense = 0, kGather = 1, kDualSilu = 2, kDenseDual = 3 };
+enum Mode { kDense = 0, kGather = 1, kDualSilu = 2, kDenseDual = 3, kDenseSplit = 4 };
 
 constexpr int kWaves = 8;
 constexpr int kBM = 128;     // weight rows per workgroup (or 256: the dense tile of gemm_sk)
@@ -159,6 +162,9 @@ struct GemmArgs {
     const int4* tiles;  // gather modes: (expert, p0, n, 0)
     const int* ntiles;
     const int* tok;     // gather modes: X row of each position
+    float* part;        // split mode: fp32 partial sums [ksplit][T][ldp]
+    int64_t ldp;
+    int ksplit, ttiles; // split mode: parts of K, token tiles
 };
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
@@ -192,7 +198,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
     const int kq = wave % KS, rq = wave / KS;
 
     // ---- tile
-    int m0, t0 = 0, nt, p0 = 0;
+    int m0, t0 = 0, nt, p0 = 0, nst = a.K / kStageK, split = 0;
+    int64_t k0 = 0;  // first k of this workgroup's part (split mode)
     const uint8_t *wA = a.w, *sA = a.s, *bA = a.b, *wB = a.w2, *sB = a.s2, *bB = a.b2;
     if constexpr (kGath) {
         // The grid covers the worst case; the first ntiles * mtiles
@@ -225,11 +232,28 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
         const int per = nwg >> 3, rem = nwg & 7, xcd = b & 7;
         const int q = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
         m0 = (q % a.mtiles) * (kDual ? BM / 2 : BM);
-        t0 = (q / a.mtiles) * BT;
+        int tt = q / a.mtiles;
+        if constexpr (MODE == kDenseSplit) {
+            // part `split` of K: whole units of 256 k, so every row's slot
+            // windows start as they do at k = 0 (Q8_0's alternate by stage)
+            split = tt / a.ttiles;
+            tt -= split * a.ttiles;
+            const int units = a.K / 256;
+            const int u0 = static_cast<int>(static_cast<int64_t>(units) * split / a.ksplit);
+            const int u1 = static_cast<int>(static_cast<int64_t>(units) * (split + 1) / a.ksplit);
+            nst = 2 * (u1 - u0);
+            k0 = 256 * static_cast<int64_t>(u0);
+            wA += Fm::kAff ? k0 / 2 : k0 / 32 * (F == WF::Q8_0 ? 34 : 18);
+            if constexpr (Fm::kAff) {
+                sA += k0 / Fm::G * 2;
+                bA += k0 / Fm::G * 2;
+            }
+        }
+        t0 = tt * BT;
         nt = min(BT, a.T - t0);
     }
     const int M = a.M, K = a.K;
-    const int nst = K / kStageK, ngr = nst / SPS;
+    const int ngr = nst / SPS;
     const uint32_t lds0 = lds_addr(lds);
 
     // ---- X sources: transfer i of this wave (i = NX*wave + ii) fills 16-byte
@@ -249,7 +273,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
         else row = tl;
         xoff[ii] = static_cast<uint32_t>(2 * (row * a.ldx + 8 * c));
     }
-    const uint16_t* xbase = kGath ? a.x : a.x + static_cast<int64_t>(t0) * a.ldx;
+    const uint16_t* xbase = kGath ? a.x : a.x + static_cast<int64_t>(t0) * a.ldx + k0;
 
     // ---- W sources.  Transfer i = 8*ii + wave of a slot (ii < CW: 3, or 5 for
     // the 256-row GGUF slot).  ii < CW - 1 are 16-byte transfers of GGUF
@@ -647,7 +671,11 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int t = 32 * (pass * PF + f) + 8 * j + 4 * h + i;
-                    if (t < nt && m < M) a.y[yrow(t) * a.ldy + m] = f2h_bits(sum[i]);
+                    if constexpr (MODE == kDenseSplit) {
+                        if (t < nt && m < M) a.part[(static_cast<int64_t>(split) * a.T + t0 + t) * a.ldp + m] = sum[i];
+                    } else {
+                        if (t < nt && m < M) a.y[yrow(t) * a.ldy + m] = f2h_bits(sum[i]);
+                    }
                 }
             }
         } else {
@@ -724,8 +752,103 @@ inline Tile pick_tile(int64_t rows, int64_t T, int64_t K, bool allow256) {
     return c128 < c64 ? Tile::k128x128 : Tile::k128x64;
 }
 
+// y[t][m..m+3] = fp16 of the K parts' partial sums, added in part order.
+template <bool VEC>
+__global__ __launch_bounds__(256) void split_sum(const float* __restrict__ part, int64_t ldp, int ksplit, int M, int T,
+                                                 uint16_t* __restrict__ y, int64_t ldy) {
+    const int64_t q = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, per = ldp / 4;
+    if (q >= per * T) return;
+    const int64_t t = q / per, m = 4 * (q % per), plane = static_cast<int64_t>(T) * ldp;
+    const float* p = part + t * ldp + m;
+    float4_t sum = *reinterpret_cast<const float4_t*>(p);
+#pragma unroll 4
+    for (int s = 1; s < ksplit; ++s) sum += *reinterpret_cast<const float4_t*>(p + s * plane);
+    uint16_t* o = y + t * ldy + m;
+    if constexpr (VEC) {
+        uint2 v;
+        v.x = f2h_bits(sum[0]) | (static_cast<uint32_t>(f2h_bits(sum[1])) << 16);
+        v.y = f2h_bits(sum[2]) | (static_cast<uint32_t>(f2h_bits(sum[3])) << 16);
+        *reinterpret_cast<uint2*>(o) = v;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (m + i < M) o[i] = f2h_bits(sum[i]);
+    }
+}
+
+// Tile shape and K parts of a dense launch that has a workspace.  A launch of
+// fewer tiles than CUs is bound by the length of one tile's K loop (its stages
+// run at 0.2-0.3 of the CU's MFMA rate, each waiting for its transfers and the
+// workgroup), while the other CUs are idle.  Parts of K give them work, for
+// one more launch and the traffic of the partial sums.  Estimated as in
+// pick_tile, with the constants fitted to launches of one round: 5 us fixed,
+// 22 us x r per 4096 of K, and for a split 4 us plus its partial sums' bytes
+// at 4 TB/s; taken where it saves 5%.  Measured, whole -> split (us): Q8_0
+// 8192 x 28672 at 100 / 256 tokens 190.5 -> 92.5 (128 tokens, 4 parts) / 209
+// -> 177 (128, 2); 8192 x 8192 at 64 / 128 60.8 -> 27.9 (64, 4) / 58.5 -> 37.3
+// (128, 4); 11008 x 4096 at 60 33.5 -> 24.5 (64, 2); Q4_0 4096 x 11008 at 128 /
+// 256 / 333 56.7 -> 27.2 (64, 4) / 57.8 -> 38.7 (128, 4) / 59.1 -> 55.1 (128,
+// 2); 4096 x 4096 at 64 24.9 -> 15.5 (64, 4); 2048 x 4096 at 512 25.4 -> 23.1
+// (64, 2).  4096 x 11008 at 512 (64.6 -> 61.9, 128 tokens, 2 parts) stays whole,
+// and so does every launch whose whole tiles fill the CUs.
+struct SplitPlan {
+    int bt = 0, parts = 1;
+};
+inline int64_t split_ld(int64_t M) { return (M + 3) / 4 * 4; }
+inline size_t split_bytes(const SplitPlan& p, int64_t M, int64_t T) {
+    return p.parts > 1 ? static_cast<size_t>(p.parts) * T * split_ld(M) * sizeof(float) : 0;
+}
+inline SplitPlan pick_split(int64_t M, int64_t T, int64_t K) {
+    const int64_t cu = cu_count(), units = K / 256;
+    if (M <= 0 || T <= 0 || K % 256 != 0) return {};
+    auto jobs = [&](int64_t bm, int64_t bt) { return (M + bm - 1) / bm * ((T + bt - 1) / bt); };
+    auto rounds = [&](int64_t n) { return static_cast<double>((n + cu - 1) / cu); };
+    const double unit = 22.0 * static_cast<double>(K) / 4096.0;
+    const double whole = std::min({rounds(jobs(128, 64)) * (5.0 + 1.1 * unit), rounds(jobs(128, 128)) * (5.0 + 1.7 * unit),
+                                   rounds(jobs(256, 128)) * (5.0 + 2.6 * unit)});
+    SplitPlan best;
+    double cost = whole * 0.95;
+    for (int bt : {128, 64})
+        for (int s = 2; s <= 8 && units / s >= 4; ++s) {
+            const double c = rounds(jobs(128, bt) * s) * (5.0 + (bt == 128 ? 1.7 : 1.1) * unit / s) + 4.0 +
+                             8.0 * s * static_cast<double>(T) * static_cast<double>(M) / 4e6;
+            if (c < cost) {
+                cost = c;
+                best.bt = bt;
+                best.parts = s;
+            }
+        }
+    return best;
+}
+
+template <WF F, int BT>
+int dense_split_gemm(GemmArgs a, const SplitPlan& p, float* part, hipStream_t stream) {
+    a.mtiles = (a.M + kBM - 1) / kBM;
+    a.ttiles = (a.T + BT - 1) / BT;
+    a.ksplit = p.parts;
+    a.part = part;
+    a.ldp = split_ld(a.M);
+    // pick_split splits only launches of few tiles, so the grid stays small
+    if (int rc = launch_sk<F, BT, kDenseSplit>(a, static_cast<unsigned>(a.mtiles) * a.ttiles * a.ksplit, stream)) return rc;
+    const int64_t threads = a.ldp / 4 * a.T;
+    const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
+    if (a.M % 4 == 0 && a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 8 == 0)
+        hipLaunchKernelGGL((split_sum<true>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
+    else
+        hipLaunchKernelGGL((split_sum<false>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
+    return check_hip(hipGetLastError(), "split_sum launch");
+}
+
 template <WF F>
-int dense_gemm_auto(const GemmArgs& a, hipStream_t stream) {
+int dense_gemm_auto(const GemmArgs& a, void* workspace, size_t bytes, hipStream_t stream) {
+    if (workspace) {
+        const SplitPlan p = pick_split(a.M, a.T, a.K);
+        const size_t need = split_bytes(p, a.M, a.T);
+        if (need > 0 && need <= bytes) {
+            float* part = static_cast<float*>(workspace);
+            return p.bt == 128 ? dense_split_gemm<F, 128>(a, p, part, stream) : dense_split_gemm<F, 64>(a, p, part, stream);
+        }
+    }
     switch (pick_tile(a.M, a.T, a.K, true)) {
         case Tile::k256x128: return dense_gemm<F, 128, 2 * kBM>(a, stream);
         case Tile::k128x128: return dense_gemm<F, 128>(a, stream);
@@ -1068,7 +1191,7 @@ int off_grid(const std::string& n, int64_t in_dim) {
 
 template <WF F>
 int run_dense(const void* w, const void* s, const void* b, const void* x, void* y, int64_t M, int64_t K, int64_t T,
-              int64_t ldx, int64_t ldy, void* stream) {
+              int64_t ldx, int64_t ldy, void* workspace, size_t bytes, void* stream) {
     GemmArgs a{};
     a.w = static_cast<const uint8_t*>(w);
     a.s = static_cast<const uint8_t*>(s);
@@ -1083,38 +1206,59 @@ int run_dense(const void* w, const void* s, const void* b, const void* x, void* 
     a.T = static_cast<int>(T);
     a.ldx = ldx;
     a.ldy = ldy;
-    const int rc = dense_gemm_auto<F>(a, as_stream(stream));
+    if (reinterpret_cast<uintptr_t>(workspace) % 16)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, "dequant_gemm: workspace must be 16-byte aligned");
+    const int rc = dense_gemm_auto<F>(a, workspace, bytes, as_stream(stream));
     return rc == GDSLLM_OK ? ok() : rc;
 }
 
 }  // namespace
 
-extern "C" int gdsllm_dequant_gemm_q8_0(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
-                                        int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+extern "C" size_t gdsllm_dequant_gemm_workspace_size(int64_t out_dim, int64_t in_dim, int64_t tokens) {
+    return split_bytes(pick_split(out_dim, tokens, in_dim), out_dim, tokens);
+}
+
+extern "C" int gdsllm_dequant_gemm_q8_0_ws(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                           int64_t tokens, int64_t ldx, int64_t ldy, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
     bool empty;
     if (int rc = check_dense("dequant_gemm_q8_0", weight, x, y, out_dim, in_dim, tokens, ldx, ldy, empty)) return rc;
     if (empty) return ok();
     if (in_dim % 256 != 0) return off_grid("dequant_gemm_q8_0", in_dim);
     if (int rc = check_q8_rows("dequant_gemm_q8_0", in_dim)) return rc;
-    return run_dense<WF::Q8_0>(weight, nullptr, nullptr, x, y, out_dim, in_dim, tokens, ldx, ldy, stream);
+    return run_dense<WF::Q8_0>(weight, nullptr, nullptr, x, y, out_dim, in_dim, tokens, ldx, ldy, workspace,
+                               workspace_bytes, stream);
 }
 
-extern "C" int gdsllm_dequant_gemm_q4_0(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
+extern "C" int gdsllm_dequant_gemm_q8_0(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
                                         int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+    return gdsllm_dequant_gemm_q8_0_ws(weight, x, y, out_dim, in_dim, tokens, ldx, ldy, nullptr, 0, stream);
+}
+
+extern "C" int gdsllm_dequant_gemm_q4_0_ws(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                           int64_t tokens, int64_t ldx, int64_t ldy, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
     bool empty;
     if (int rc = check_dense("dequant_gemm_q4_0", weight, x, y, out_dim, in_dim, tokens, ldx, ldy, empty)) return rc;
     if (empty) return ok();
     if (in_dim % 256 == 0)
-        return run_dense<WF::Q4_0>(weight, nullptr, nullptr, x, y, out_dim, in_dim, tokens, ldx, ldy, stream);
+        return run_dense<WF::Q4_0>(weight, nullptr, nullptr, x, y, out_dim, in_dim, tokens, ldx, ldy, workspace,
+                                   workspace_bytes, stream);
     // off the split-K grid: one Q4_0 block per K step
     const int r = dequant_gemm_q4_0_blockwise(weight, x, y, static_cast<int>(out_dim), static_cast<int>(in_dim),
                                               static_cast<int>(tokens), ldx, ldy, as_stream(stream));
     return r == GDSLLM_OK ? ok() : r;
 }
 
-extern "C" int gdsllm_dequant_gemm_affine_q4(const void* weight, const void* scales, const void* biases, const void* x,
-                                             void* y, int64_t out_dim, int64_t in_dim, int64_t group_size,
-                                             int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+extern "C" int gdsllm_dequant_gemm_q4_0(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                        int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+    return gdsllm_dequant_gemm_q4_0_ws(weight, x, y, out_dim, in_dim, tokens, ldx, ldy, nullptr, 0, stream);
+}
+
+extern "C" int gdsllm_dequant_gemm_affine_q4_ws(const void* weight, const void* scales, const void* biases,
+                                                const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                                int64_t group_size, int64_t tokens, int64_t ldx, int64_t ldy,
+                                                void* workspace, size_t workspace_bytes, void* stream) {
     const std::string n = "dequant_gemm_affine_q4";
     if (group_size <= 0 || group_size % 8 != 0)
         return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": group_size must be a positive multiple of 8");
@@ -1131,10 +1275,20 @@ extern "C" int gdsllm_dequant_gemm_affine_q4(const void* weight, const void* sca
     if (reinterpret_cast<uintptr_t>(scales) % sal || reinterpret_cast<uintptr_t>(biases) % sal)
         return set_error(GDSLLM_ERR_UNSUPPORTED, n + ": scales/biases must be " + std::to_string(sal) + "-byte aligned");
     switch (group_size) {
-        case 32: return run_dense<WF::AFF32>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, stream);
-        case 64: return run_dense<WF::AFF64>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, stream);
-        default: return run_dense<WF::AFF128>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, stream);
+        case 32: return run_dense<WF::AFF32>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, workspace,
+                                                  workspace_bytes, stream);
+        case 64: return run_dense<WF::AFF64>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, workspace,
+                                                  workspace_bytes, stream);
+        default: return run_dense<WF::AFF128>(weight, scales, biases, x, y, out_dim, in_dim, tokens, ldx, ldy, workspace,
+                                                  workspace_bytes, stream);
     }
+}
+
+extern "C" int gdsllm_dequant_gemm_affine_q4(const void* weight, const void* scales, const void* biases, const void* x,
+                                             void* y, int64_t out_dim, int64_t in_dim, int64_t group_size,
+                                             int64_t tokens, int64_t ldx, int64_t ldy, void* stream) {
+    return gdsllm_dequant_gemm_affine_q4_ws(weight, scales, biases, x, y, out_dim, in_dim, group_size, tokens, ldx, ldy,
+                                            nullptr, 0, stream);
 }
 
 extern "C" size_t gdsllm_moe_prefill_workspace_size(int64_t tokens, int64_t top_k, int64_t ffn_dim, int64_t hidden,

@@ -328,6 +328,24 @@ int gdsllm_dequant_gemm_affine_q4(const void* weight, const void* scales, const 
                                   const void* x, void* y, int64_t out_dim, int64_t in_dim,
                                   int64_t group_size, int64_t tokens, int64_t ldx, int64_t ldy,
                                   void* stream);
+/* The same three with a device workspace (16-byte aligned): a launch whose
+ * tiles leave compute units idle (70B down_proj over 100 tokens: 128 of 256)
+ * splits K over workgroups, keeps their fp32 partial sums there and adds them
+ * in a fixed order in a second launch.  Results differ from the entries
+ * above by fp32 reassociation only.  With a null or smaller workspace than
+ * gdsllm_dequant_gemm_workspace_size (0: no split) they are those entries.  */
+size_t gdsllm_dequant_gemm_workspace_size(int64_t out_dim, int64_t in_dim, int64_t tokens);
+int gdsllm_dequant_gemm_q4_0_ws(const void* weight, const void* x, void* y, int64_t out_dim,
+                                int64_t in_dim, int64_t tokens, int64_t ldx, int64_t ldy,
+                                void* workspace, size_t workspace_bytes, void* stream);
+int gdsllm_dequant_gemm_q8_0_ws(const void* weight, const void* x, void* y, int64_t out_dim,
+                                int64_t in_dim, int64_t tokens, int64_t ldx, int64_t ldy,
+                                void* workspace, size_t workspace_bytes, void* stream);
+int gdsllm_dequant_gemm_affine_q4_ws(const void* weight, const void* scales, const void* biases,
+                                     const void* x, void* y, int64_t out_dim, int64_t in_dim,
+                                     int64_t group_size, int64_t tokens, int64_t ldx, int64_t ldy,
+                                     void* workspace, size_t workspace_bytes, void* stream);
+
 /* The MLP input of a prefill chunk in one launch: h[t][r] =
  * fp16(fp16(silu(g)) * u) with g = fp16(sum_k x[t][k] * gate[r][k]) and u
  * likewise for up (GGUF Q4_0 / Q8_0 [ffn_dim][in_dim]; g and u are the bits

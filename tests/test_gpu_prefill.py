@@ -467,3 +467,48 @@ def test_dequant_gemm_gate_up_silu(gpu, fmt, T, F, K):
     rel = float(np.linalg.norm(hk[rows] - h_oracle) / np.linalg.norm(h_oracle))
     print(f"gate_up_silu {fmt} T{T} {F}x{K}: rel L2 {rel:.2e}")
     assert rel <= oq.GEMV_REL_L2, f"h end-to-end rel L2 {rel:.3e}"
+
+
+# (T, M, K) of the *_ws entries: one or several parts of K with equal and
+# unequal unit counts, rows off the 128 grid and off the 4-row vector store,
+# ragged token tiles; the last does not split (its tiles fill the chip).
+SPLIT_CASES = [(1, 256, 8192), (37, 1000, 5888), (64, 389, 28672), (100, 1026, 11008), (130, 512, 8448),
+               (512, 11008, 256)]
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "affine32", "affine64", "affine128"])
+@pytest.mark.parametrize("T,M,K", SPLIT_CASES, ids=[f"T{t}_{m}x{k}" for t, m, k in SPLIT_CASES])
+def test_dequant_gemm_split_k(gpu, fmt, T, M, K):
+    """K split over workgroups with the partial sums in the workspace, against
+    the oracle; a null workspace takes the whole-K launch, equal within fp32
+    reassociation (one fp16 ulp plus 2^-16 of ||w_r * x||); bytes past the
+    workspace and columns past the rows stay as they were."""
+    x = syn.activations(T, K, gen(5801 + T))
+    xd = x.to(gpu)
+    ldy = M + 3
+    need = capi().gdsllm_dequant_gemm_workspace_size(M, K, T)
+    assert (need > 0) == (M < 11008)
+    ws = torch.full((need + 256,), 0xA5, dtype=torch.uint8, device=gpu)
+    ys = [torch.full((T, ldy), 7.0, dtype=torch.float16, device=gpu) for _ in range(2)]
+    for y, wp, nbytes in ((ys[0], ptr(ws), need), (ys[1], None, 0)):
+        if fmt.startswith("affine"):
+            g = int(fmt[6:])
+            words, scales, biases = syn.affine_q4_weights([M, K], g, gen(5802 + M + g))
+            deq = affine_dequant_np(words, scales, biases, g).reshape(M, K)
+            wd, sd, bd = words.to(gpu), scales.to(gpu), biases.to(gpu)
+            check(capi().gdsllm_dequant_gemm_affine_q4_ws(ptr(wd), ptr(sd), ptr(bd), ptr(xd), ptr(y), M, K, g, T, K,
+                                                          ldy, wp, nbytes, stream()))
+        else:
+            w = (syn.q4_0_weights if fmt == "q4_0" else syn.q8_0_weights)(M, K, gen(5800 + M + K))
+            deq = (oq.dequant_q4_0 if fmt == "q4_0" else oq.dequant_q8_0)(to_np(w)).reshape(M, K)
+            wd = w.to(gpu)
+            fn = capi().gdsllm_dequant_gemm_q4_0_ws if fmt == "q4_0" else capi().gdsllm_dequant_gemm_q8_0_ws
+            check(fn(ptr(wd), ptr(xd), ptr(y), M, K, T, K, ldy, wp, nbytes, stream()))
+        torch.cuda.synchronize()
+    a, b = (to_np(y)[:, :M].copy() for y in ys)
+    assert_gemv_close(a, deq, to_np(x), f"{fmt} split gemm T{T} {M}x{K}")
+    assert all((to_np(y)[:, M:] == 7.0).all() for y in ys), "columns past the rows were written"
+    assert bool((ws[need:] == 0xA5).all()), "bytes past the workspace were written"
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    bound = oq.fp16_ulp(np.maximum(np.abs(a), np.abs(b))) + oq.row_norms(deq, to_np(x)) * 2.0 ** -16
+    assert (np.abs(a - b) <= bound).all()
