@@ -1508,31 +1508,39 @@ int launch_q4_codes(const void* w, const uint16_t* x, uint16_t* y, int M, int K,
     return check_hip(hipGetLastError(), "gguf_gemv_q4_codes launch");
 }
 
-// ---- Q4_0 codes on MFMA with x held in registers (in_dim <= 8192) ----------
+// ---- Codes on MFMA with x held in registers --------------------------------
 //
-// Same operands and arithmetic as gguf_gemv_q4_codes, different data
-// movement.  Wave w of a 16-wave workgroup always takes super-blocks w and
-// w+16 of K, for every 16-row tile the workgroup owns, so its slice of x (up
-// to 2 super-blocks x 8 batch rows, 8 KiB) is loaded once instead of once per
-// tile.  LDS then holds weights only: 4 stage slots per wave, so a tile's
-// whole K is in flight at once.  The x slice comes in by LDS DMA (2 batch rows
+// Q4_0 (in_dim <= 8192): same operands and arithmetic as gguf_gemv_q4_codes,
+// different data movement.  Q8_0 (in_dim <= 8192): the same with the codes'
+// exact values q as the weight operand and the block scale applied to the
+// fp32 product sums.  Wave w of a 16-wave workgroup always takes super-blocks
+// w and w+16 of K, for every 16-row tile the workgroup owns, so its slice of x
+// (up to 2 super-blocks x 8 batch rows, 8 KiB) is loaded once instead of once
+// per tile.  LDS then holds weights only: 4 stage slots per wave (Q8_0: 2, of
+// twice the bytes), so a tile's whole K is in flight at once.  The x slice comes in by LDS DMA (2 batch rows
 // x 512 contiguous bytes per transfer) into the wave's slots and is read into
 // registers before the first weights are issued; register loads straight
 // from HBM gathered 8 batch rows per instruction and took ~4 us longer per
 // launch.
 namespace bx {
 constexpr int kRT = 16;  // rows per tile
-constexpr int kNWD = (kRT * 9 + 63) / 64;                  // weight transfers per stage (3)
-constexpr int kLastLanes = kRT * 9 - 64 * (kNWD - 1);      // lanes of the last one (16)
-constexpr int kSlotBytes = kRT * 144;                      // one super-block of the tile's rows
 // WV waves per workgroup, at most NSB super-blocks of K per wave, NS stage
-// slots per wave.
-template <int WV, int NSB, int NS>
+// slots per wave; XSEP: the x slice comes into LDS of its own.
+template <Fmt F, int WV, int NSB, int NS, bool XSEP = false>
 struct Cfg {
+    static constexpr Fmt kFmt = F;
+    static constexpr int kSb = Layout<F>::kSbBytes;                // a row's super-block
+    static constexpr int kCh = kSb / 16;                           // its 16-byte chunks (9, 17)
+    static constexpr int kNWD = (kRT * kCh + 63) / 64;             // weight transfers per stage (3, 5)
+    static constexpr int kLastLanes = kRT * kCh - 64 * (kNWD - 1); // lanes of the last one (16)
+    static constexpr int kSlotBytes = kRT * kSb;                   // one super-block of the tile's rows
     static constexpr int kWaves = WV, kNSB = NSB, kNS = NS;
     static constexpr int kRedBytes = WV * 8 * kRT * 4;  // one tile's partial sums
-    static constexpr int kLdsBytes = WV * NS * kSlotBytes + 2 * kRedBytes;
-    static_assert(NS * kSlotBytes >= NSB * 4096, "the x slice is staged in the wave's slots");
+    static constexpr bool kXSep = XSEP;
+    static constexpr int kXBytes = NSB * 4096;  // a wave's x slice
+    static constexpr int kXOff = WV * NS * kSlotBytes + 2 * kRedBytes;
+    static constexpr int kLdsBytes = kXOff + (XSEP ? WV * kXBytes : 0);
+    static_assert(XSEP || NS * kSlotBytes >= kXBytes, "the x slice is staged in the wave's slots");
     static_assert(kLdsBytes <= 160 * 1024, "LDS of one compute unit");
 };
 // 16 waves x 2 super-blocks (in_dim <= 8192), 4 slots: a 16-row tile's whole
@@ -1541,7 +1549,7 @@ struct Cfg {
 // Measured against 8 waves x 4 super-blocks with 8 slots and the corrections
 // kept in registers (batch 8, us): 28672x8192 31.7 / 34.3, 13003x4096
 // 13.7 / 15.8, 9000x5120 12.2 / 14.2.
-using Tall = Cfg<16, 2, 4>;
+using Tall = Cfg<Fmt::Q4_0, 16, 2, 4>;
 // in_dim <= 4096: 8 waves x 2 super-blocks, 4 slots (80 KiB, two workgroups
 // per CU, each with its own barrier) where there are at least two 16-row
 // tiles per CU.  Batch 3 / 4 / 8 against Tall, us: 11008x4096 9.5 / 9.6 /
@@ -1549,7 +1557,23 @@ using Tall = Cfg<16, 2, 4>;
 // 13.9 / 13.9 / 14.4; the 7B q/k/v group 10.0 / 10.3 / 10.8 against 11.6 /
 // 11.8 / 12.2 and gate/up pair 17.4 / 17.5 / 18.0 against 19.9 / 20.0 /
 // 20.4; with one tile per CU (4096x4096 at batch 3) 5.45 against 5.17.
-using Half = Cfg<8, 2, 4>;
+using Half = Cfg<Fmt::Q4_0, 8, 2, 4>;
+// Q8_0: the waves' shares of K go by in_dim alone, so a matrix has the same
+// bits alone and in a group.  in_dim <= 4096: Half's split, 2 slots (78 KiB,
+// two workgroups per CU); with at most one tile per CU the x slice has LDS of
+// its own (140 KiB), so the tile's weights are in flight while x comes in.
+// in_dim <= 8192: Tall's split with 2 slots.  Both wave counts with twice the
+// slots, 4 waves x 4 slots, and 8 waves x 4 super-blocks were no faster at any
+// of 15 shapes.  Against gguf_gemv_mfma, which takes x in with every stage (as
+// many bytes as its weights) and launches each matrix by itself, batch 3 / 8,
+// us: 11008x4096 15.1 / 15.9 -> 13.7 / 14.3, 32000x4096 35.2 / 38.3 -> 29.8 /
+// 30.4, 28672x8192 58.1 / 66.2 -> 49.8 / 51.4, 14336x5120 22.8 / 25.7 -> 22.4 /
+// 22.9, 1024x8192 8.8 / 10.2 -> 7.5 / 9.5, 8192x8192 19.1 / 20.1 -> 19.6 / 20.0.
+// Past 8192 a wave's x slice is longer than its weights' gain: 4096x11008 14.3
+// / 16.8 against 15.7 / 19.4 with 8 waves x 8 super-blocks, so those keep it.
+using Q8Half = Cfg<Fmt::Q8_0, 8, 2, 2>;
+using Q8Few = Cfg<Fmt::Q8_0, 8, 2, 2, true>;
+using Q8Tall = Cfg<Fmt::Q8_0, 16, 2, 2>;
 
 // Where a launch reads weights and writes results.  MODE 0: one matrix
 // (w[0], y[0], m[0]); 1: up to 4 matrices of the same in_dim sharing x, whose
@@ -1598,36 +1622,38 @@ __device__ __forceinline__ Tile tile_of(const Target& tg, int t) {
 }  // namespace bx
 
 template <class C, int MODE>
-__global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Target tg,
+__global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_xreg(const bx::Target tg,
                                                                     const uint16_t* __restrict__ X, int K, int nb,
                                                                     int64_t ldx) {
-    constexpr int RT = bx::kRT, NRG = RT / 8, NS = C::kNS;
+    constexpr Fmt F = C::kFmt;
+    static_assert(F == Fmt::Q4_0 || MODE != 2, "gate/up pairs are Q4_0");
+    constexpr int RT = bx::kRT, NRG = RT / 8, NS = C::kNS, kCh = C::kCh, kSb = C::kSb;
     // transfers per stage: 3 (16 rows of one matrix); pairing: 2 per matrix
     // (chunks 0-63 of the 8 rows, then chunks 64-71 on 8 lanes)
-    constexpr int NWD = MODE == 2 ? 4 : bx::kNWD;
+    constexpr int NWD = MODE == 2 ? 4 : C::kNWD;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int S = K >> 8;
-    const uint32_t row_bytes = static_cast<uint32_t>(S) * 144u;
+    const uint32_t row_bytes = static_cast<uint32_t>(S) * kSb;
     const int ntiles = tg.tile_end[kMaxGroup - 1];
     const int T = (ntiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
     const int nst = S > wave ? (S - 1 - wave) / C::kWaves + 1 : 0;  // super-blocks of this wave (<= NSB)
     const int Q = T * nst;
     const uint32_t lds0 = lds_addr(lds);
-    const uint32_t slot0 = lds0 + wave * NS * bx::kSlotBytes;
-    float* red0 = reinterpret_cast<float*>(lds + C::kWaves * NS * bx::kSlotBytes);
+    const uint32_t slot0 = lds0 + wave * NS * C::kSlotBytes;
+    float* red0 = reinterpret_cast<float*>(lds + C::kWaves * NS * C::kSlotBytes);
 
-    // weight transfer j: chunk c = 64j + lane = row c / 9, chunk c % 9 of the
+    // weight transfer j: chunk c = 64j + lane = row c / kCh, chunk c % kCh of the
     // row's super-block (rows past the tile's last valid row read that row).
     // Pairing: chunks of one matrix's 8 rows, c = lane, then c = 64 + lane.
     constexpr int NOFF = MODE == 2 ? 2 : NWD;
-    constexpr int kChunks = MODE == 2 ? 72 : RT * 9;
+    constexpr int kChunks = MODE == 2 ? 72 : RT * kCh;
     auto w_offsets = [&](int nrows, uint32_t (&off)[NOFF]) {
 #pragma unroll
         for (int j = 0; j < NOFF; ++j) {
             const int c = min(64 * j + lane, kChunks - 1);
-            const int r = c / 9;
-            off[j] = static_cast<uint32_t>(min(r, nrows - 1)) * row_bytes + 16u * static_cast<uint32_t>(c - 9 * r);
+            const int r = c / kCh;
+            off[j] = static_cast<uint32_t>(min(r, nrows - 1)) * row_bytes + 16u * static_cast<uint32_t>(c - kCh * r);
         }
     };
     uint32_t woff_full[NOFF];
@@ -1635,10 +1661,10 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
 
     int ii = 0, ss = 0, qs = 0;  // next stage to issue: tile ii, super-block step ss, slot qs
     auto issue = [&]() {
-        const uint32_t slot = slot0 + qs * bx::kSlotBytes;
+        const uint32_t slot = slot0 + qs * C::kSlotBytes;
         const int sb = wave + C::kWaves * ss;
         const bx::Tile tl = bx::tile_of<MODE>(tg, static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) * ii);
-        const int64_t at = static_cast<int64_t>(tl.row0) * row_bytes + 144 * sb;
+        const int64_t at = static_cast<int64_t>(tl.row0) * row_bytes + kSb * sb;
         uint32_t woff[NOFF];
         const int nrows = min(MODE == 2 ? RT / 2 : RT, tl.m - tl.row0);
         if (nrows == (MODE == 2 ? RT / 2 : RT)) {
@@ -1657,7 +1683,7 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
             const uint8_t* wb = tl.w0 + at;
 #pragma unroll
             for (int j = 0; j < NWD - 1; ++j) dma16_asm(woff[j], wb, slot + 1024 * j);
-            if (lane < bx::kLastLanes) dma16_asm(woff[NWD - 1], wb, slot + 1024 * (NWD - 1));
+            if (lane < C::kLastLanes) dma16_asm(woff[NWD - 1], wb, slot + 1024 * (NWD - 1));
         }
         if (++ss == nst) {
             ss = 0;
@@ -1668,8 +1694,16 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
 
     // per-lane operand geometry, as in gguf_gemv_q4_codes
     const int g = lane >> 4, j = lane & 15, par = j >> 3;
-    const uint32_t wrd = 144 * (j & 7) + (par ? 20 : 0) + 4 * g;
-    const uint32_t drd = 144 * (j & 7) + 18 * par;
+    // (Q8_0: qs dwords g and 4 + g of the block, shifted by 2 in even blocks)
+    const uint32_t wrd = kSb * (j & 7) + (par ? Layout<F>::kBlockBytes + 2 : 0) + 4 * g;
+    const uint32_t drd = kSb * (j & 7) + Layout<F>::kBlockBytes * par;
+    const uint32_t sh8 = par ? 0u : 2u;
+    uint32_t c64 = 0x64646464u;
+    asm volatile("" : "+v"(c64));
+    const half2_t off_q8 = {static_cast<half_t>(-1152.0f), static_cast<half_t>(-1152.0f)};
+    auto q8_pair = [&](uint32_t v, uint32_t sel) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(c64, v, sel)) + off_q8);
+    };
     const uint32_t sel01 = par ? 0x0C010C00u : 0x0C030C02u;
     const uint32_t sel23 = par ? 0x0C030C02u : 0x0C050C04u;
     const NibUnpack nu;
@@ -1727,8 +1761,10 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
     // nb <= 4; the super-blocks past this wave's last repeat it), then into
     // registers.
     half8_t xa[C::kNSB][4];
+    int issued = min(Q, NS);  // stages of weights issued
     {
         const int nxt = nb <= 4 ? 2 : 4;
+        const uint32_t xs = C::kXSep ? lds0 + C::kXOff + wave * C::kXBytes : slot0;
 #pragma unroll
         for (int s2 = 0; s2 < C::kNSB; ++s2) {
             const int sb = wave + C::kWaves * min(s2, nst - 1);
@@ -1737,13 +1773,21 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
                 if (jj >= nxt) break;
                 const int tr = min(2 * jj + (lane >> 5), nb - 1);
                 dma16_asm(static_cast<uint32_t>(2 * (tr * ldx + 8 * (lane & 31))), X + 256 * sb,
-                          slot0 + 4096 * s2 + 1024 * jj);
+                          xs + 4096 * s2 + 1024 * jj);
             }
         }
-        wait_vmcnt_asm<0>();
+        if constexpr (C::kXSep) {
+            // x went out first: wait for all but the weights' transfers
+            static_assert(NS == 2, "one or two stages issued");
+            for (int q = 0; q < issued; ++q) issue();
+            if (issued == 2) wait_vmcnt_asm<2 * NWD>();
+            else wait_vmcnt_asm<NWD>();
+        } else {
+            wait_vmcnt_asm<0>();
+        }
         // lane (g, j): batch row j & 7 of block 2p + par, elements 4g.. and 16+4g..
         const int t = min(j & 7, nb - 1);
-        const uint8_t* xl = lds + (slot0 - lds0) + (t >> 1) * 1024 + (t & 1) * 512 + 2 * (32 * par + 4 * g);
+        const uint8_t* xl = lds + (xs - lds0) + (t >> 1) * 1024 + (t & 1) * 512 + 2 * (32 * par + 4 * g);
 #pragma unroll
         for (int s2 = 0; s2 < C::kNSB; ++s2)
 #pragma unroll
@@ -1755,8 +1799,8 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
         // the reads have returned before transfers overwrite the slots
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    int issued = min(Q, NS);  // stages of weights issued
-    for (int q = 0; q < issued; ++q) issue();
+    if constexpr (!C::kXSep)
+        for (int q = 0; q < issued; ++q) issue();
 
     const half8_t kneg = {static_cast<half_t>(-1032.0f), static_cast<half_t>(-1032.0f), static_cast<half_t>(-1032.0f),
                           static_cast<half_t>(-1032.0f), static_cast<half_t>(-72.0f),   static_cast<half_t>(-72.0f),
@@ -1779,23 +1823,34 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
                     case 6: wait_vmcnt_asm<6 * NWD>(); break;
                     default: wait_vmcnt_asm<(NS - 1) * NWD>(); break;
                 }
-                const uint8_t* sl = lds + (slot0 - lds0) + cslot * bx::kSlotBytes;
+                const uint8_t* sl = lds + (slot0 - lds0) + cslot * C::kSlotBytes;
 #pragma unroll
                 for (int p = 0; p < 4; ++p)
-                    dc[p] = kCodesExact ? float4_t{0.f, 0.f, 0.f, 0.f}
+                    dc[p] = kCodesExact || F == Fmt::Q8_0 ? float4_t{0.f, 0.f, 0.f, 0.f}
                                         : __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s2][p], kneg,
                                                                                  float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
                 for (int rg = 0; rg < NRG; ++rg)
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
-                        const uint8_t* wr = sl + 1152 * rg + 36 * p;
+                        const uint8_t* wr = sl + 8 * kSb * rg + 2 * Layout<F>::kBlockBytes * p;
                         const uint32_t d0 = *reinterpret_cast<const uint32_t*>(wr + wrd);
                         const uint32_t d1 = *reinterpret_cast<const uint32_t*>(wr + wrd + 4);
                         const half_t dv = __builtin_bit_cast(half_t, *reinterpret_cast<const uint16_t*>(wr + drd));
-                        const uint32_t p01 = __builtin_amdgcn_perm(d1, d0, sel01);
-                        const uint32_t p23 = __builtin_amdgcn_perm(d1, d0, sel23);
-                        const half8_t wbv = codes_operand(p01, p23, nu, kneg);
+                        half8_t wbv;
+                        if constexpr (F == Fmt::Q4_0) {
+                            const uint32_t p01 = __builtin_amdgcn_perm(d1, d0, sel01);
+                            const uint32_t p23 = __builtin_amdgcn_perm(d1, d0, sel23);
+                            wbv = codes_operand(p01, p23, nu, kneg);
+                        } else {
+                            // bytes under an 0x64 exponent byte are 1024 + (q + 128)
+                            const uint32_t d2 = *reinterpret_cast<const uint32_t*>(wr + wrd + 16);
+                            const uint32_t d3 = *reinterpret_cast<const uint32_t*>(wr + wrd + 20);
+                            const uint32_t q0 = __builtin_amdgcn_alignbyte(d1, d0, sh8) ^ 0x80808080u;
+                            const uint32_t q1 = __builtin_amdgcn_alignbyte(d3, d2, sh8) ^ 0x80808080u;
+                            wbv = __builtin_bit_cast(half8_t, make_uint4(q8_pair(q0, 0x04010400u), q8_pair(q0, 0x04030402u),
+                                                                         q8_pair(q1, 0x04010400u), q8_pair(q1, 0x04030402u)));
+                        }
                         const float4_t D = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[s2][p], wbv, dc[p], 0, 0, 0);
                         const float dsc = static_cast<float>(dv);
 #pragma unroll
@@ -1816,17 +1871,17 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_q4_xreg(const bx::Ta
 }
 
 template <class C, int MODE>
-int launch_q4_xreg(const bx::Target& tg, const uint16_t* x, int K, int64_t batch, int64_t ldx, hipStream_t stream) {
+int launch_xreg_cfg(const bx::Target& tg, const uint16_t* x, int K, int64_t batch, int64_t ldx, hipStream_t stream) {
     constexpr size_t lds = C::kLdsBytes;
-    const void* fn = reinterpret_cast<const void*>(&gguf_gemv_q4_xreg<C, MODE>);
+    const void* fn = reinterpret_cast<const void*>(&gguf_gemv_xreg<C, MODE>);
     if (int rc = prepare_lds(fn, lds)) return rc;
     const int tiles = tg.tile_end[kMaxGroup - 1];
     const int resident = blocks_per_cu(fn, lds, C::kWaves * 64) * cu_count();
-    if (resident < 1) return set_error(GDSLLM_ERR_UNSUPPORTED, "gguf_gemv_q4_xreg: no workgroup fits a compute unit");
+    if (resident < 1) return set_error(GDSLLM_ERR_UNSUPPORTED, "gguf_gemv_xreg: no workgroup fits a compute unit");
     const int grid = std::min(tiles, resident);
-    hipLaunchKernelGGL((gguf_gemv_q4_xreg<C, MODE>), dim3(grid), dim3(C::kWaves * 64), lds, stream, tg, x, K,
+    hipLaunchKernelGGL((gguf_gemv_xreg<C, MODE>), dim3(grid), dim3(C::kWaves * 64), lds, stream, tg, x, K,
                        static_cast<int>(batch), ldx);
-    return check_hip(hipGetLastError(), "gguf_gemv_q4_xreg launch");
+    return check_hip(hipGetLastError(), "gguf_gemv_xreg launch");
 }
 
 // Which configuration a launch takes: Half for in_dim <= 4096 with at least
@@ -1838,8 +1893,19 @@ inline bool xreg_half(int K, int64_t tiles16) { return K <= 4096 && tiles16 >= 2
 template <int MODE>
 int launch_xreg(const bx::Target& tg, const uint16_t* x, int K, int64_t batch, int64_t ldx, int64_t tiles16,
                 hipStream_t stream) {
-    return xreg_half(K, tiles16) ? launch_q4_xreg<bx::Half, MODE>(tg, x, K, batch, ldx, stream)
-                                 : launch_q4_xreg<bx::Tall, MODE>(tg, x, K, batch, ldx, stream);
+    return xreg_half(K, tiles16) ? launch_xreg_cfg<bx::Half, MODE>(tg, x, K, batch, ldx, stream)
+                                 : launch_xreg_cfg<bx::Tall, MODE>(tg, x, K, batch, ldx, stream);
+}
+
+// Largest in_dim of the x-in-registers kernel.
+constexpr int kXregMaxK = 8192;
+
+// Q8_0 at batch 3-8, in_dim % 256 == 0 up to kXregMaxK.
+template <int MODE>
+int launch_q8_xreg(const bx::Target& tg, const uint16_t* x, int K, int64_t batch, int64_t ldx, hipStream_t stream) {
+    if (K > 4096) return launch_xreg_cfg<bx::Q8Tall, MODE>(tg, x, K, batch, ldx, stream);
+    return tg.tile_end[kMaxGroup - 1] <= cu_count() ? launch_xreg_cfg<bx::Q8Few, MODE>(tg, x, K, batch, ldx, stream)
+                                                    : launch_xreg_cfg<bx::Q8Half, MODE>(tg, x, K, batch, ldx, stream);
 }
 
 // Target of one matrix: tiles of 16 rows.
@@ -2270,6 +2336,10 @@ int gemv(const char* name, const void* w, const void* x, void* y, int64_t out_di
     }
     if (fast && batch >= 3 && K <= (1 << 20) && x_al16) {
         // Q8_0 (Q4_0 took the code kernels above)
+        if (F == Fmt::Q8_0 && K <= kXregMaxK && 2 * (7 * ldx + K) < (int64_t{1} << 31)) {
+            const int rc2 = launch_q8_xreg<0>(xreg_single(w, y, M, ldy), xp, K, batch, ldx, s);
+            return rc2 == GDSLLM_OK ? ok() : rc2;
+        }
         const int rc2 = launch_mfma<F, 1>(w, xp, yp, M, K, batch, ldx, ldy, s);
         return rc2 == GDSLLM_OK ? ok() : rc2;
     }
@@ -2302,10 +2372,10 @@ int gemv(const char* name, const void* w, const void* x, void* y, int64_t out_di
 }
 
 // Batch 3-8 launches of the x-in-registers kernel over several matrices
-// (groups, gate/up pairs): in_dim a multiple of 256 up to 8192 (one slice of
-// x per wave), 16-byte aligned weights and x rows, x offsets within 2^31.
+// (groups, gate/up pairs): in_dim a multiple of 256 up to kXregMaxK (one slice
+// of x per wave), 16-byte aligned weights and x rows, x offsets within 2^31.
 bool xreg_fits(const uint8_t* const* w, int n, const void* x, int64_t K, int64_t batch, int64_t ldx) {
-    if (batch < 3 || K % 256 != 0 || K > 8192 || reinterpret_cast<uintptr_t>(x) % 16 != 0 || ldx % 8 != 0 ||
+    if (batch < 3 || K % 256 != 0 || K > kXregMaxK || reinterpret_cast<uintptr_t>(x) % 16 != 0 || ldx % 8 != 0 ||
         2 * (7 * ldx + K) >= (int64_t{1} << 31))
         return false;
     for (int i = 0; i < n; ++i)
@@ -2314,7 +2384,7 @@ bool xreg_fits(const uint8_t* const* w, int n, const void* x, int64_t K, int64_t
 }
 
 // n matrices sharing x (q/k/v of one layer): one launch when the row-span
-// kernel (batch 1-2) or the x-in-registers kernel (Q4_0, batch 3-8) serves
+// kernel (batch 1-2) or the x-in-registers kernel (batch 3-8) serves
 // the shape, else one GEMV per matrix.
 template <Fmt F>
 int gemv_group(const char* name, int n, const void* const* w, void* const* y, const int64_t* out_dims,
@@ -2343,7 +2413,7 @@ int gemv_group(const char* name, int n, const void* const* w, void* const* y, co
     const int rc = n == 1 ? try_rows<F, 0>(tg, x, static_cast<int>(in_dim), batch, ldx, as_stream(stream))
                           : try_rows<F, 1>(tg, x, static_cast<int>(in_dim), batch, ldx, as_stream(stream));
     if (rc != -1) return rc == GDSLLM_OK ? ok() : rc;
-    if (F == Fmt::Q4_0 && n > 1 && xreg_fits(tg.w, n, x, in_dim, batch, ldx)) {
+    if (n > 1 && xreg_fits(tg.w, n, x, in_dim, batch, ldx)) {
         // batch 3-8: the x-in-registers kernel over the matrices' 16-row tiles
         bx::Target xt{};
         int tiles = 0;
@@ -2353,8 +2423,10 @@ int gemv_group(const char* name, int n, const void* const* w, void* const* y, co
             xt.tile_end[i] = tiles;
         }
         for (int i = n; i < kMaxGroup; ++i) xt.tile_end[i] = tiles;
-        const int rc2 = launch_xreg<1>(xt, static_cast<const uint16_t*>(x), static_cast<int>(in_dim), batch, ldx,
-                                       tiles, as_stream(stream));
+        const auto* xp = static_cast<const uint16_t*>(x);
+        const int K = static_cast<int>(in_dim);
+        const int rc2 = F == Fmt::Q4_0 ? launch_xreg<1>(xt, xp, K, batch, ldx, tiles, as_stream(stream))
+                                       : launch_q8_xreg<1>(xt, xp, K, batch, ldx, as_stream(stream));
         return rc2 == GDSLLM_OK ? ok() : rc2;
     }
     for (int i = 0; i < n; ++i)
