@@ -506,8 +506,9 @@ std::optional<torch::Tensor> moe_step_affine_q4(torch::Tensor x, std::vector<Aff
 
 // The partial-sum workspace of a prefill GEMM that splits K, from torch's
 // allocator on the current stream (undefined where the library does not split).
-torch::Tensor gemm_workspace(int64_t out_dim, int64_t in_dim, int64_t tokens, int dev) {
-    const auto bytes = static_cast<int64_t>(gdsllm_dequant_gemm_workspace_size(out_dim, in_dim, tokens));
+torch::Tensor gemm_workspace(int64_t out_dim, int64_t in_dim, int64_t tokens, int dev, bool gate_up = false) {
+    const auto bytes = static_cast<int64_t>((gate_up ? gdsllm_dequant_gemm_gate_up_silu_workspace_size
+                                                     : gdsllm_dequant_gemm_workspace_size)(out_dim, in_dim, tokens));
     if (bytes == 0) return {};
     return torch::empty({bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, dev));
 }
@@ -570,9 +571,10 @@ std::optional<torch::Tensor> fused_gate_up_silu_gemm(const Handle& gate, const H
     auto out_shape = xf.sizes().vec();
     out_shape.back() = out_dim;
     torch::Tensor h = torch::empty(out_shape, fp16_on(dev));
-    const int rc = (q4 ? gdsllm_dequant_gemm_gate_up_silu_q4_0 : gdsllm_dequant_gemm_gate_up_silu_q8_0)(
+    torch::Tensor ws = gemm_workspace(out_dim, in_dim, tokens, dev, true);
+    const int rc = (q4 ? gdsllm_dequant_gemm_gate_up_silu_q4_0_ws : gdsllm_dequant_gemm_gate_up_silu_q8_0_ws)(
         at_offset(gate, gate_offset), at_offset(up, up_offset), xf.data_ptr(), h.data_ptr(), out_dim, in_dim, tokens,
-        in_dim, out_dim, OnDevice(dev).stream());
+        in_dim, out_dim, ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, OnDevice(dev).stream());
     if (rc == GDSLLM_ERR_UNSUPPORTED) return std::nullopt;
     check(rc, where);
     return h;
@@ -604,6 +606,37 @@ std::optional<torch::Tensor> fused_affine_q4_gemm(const Handle& h, torch::Tensor
     if (rc == GDSLLM_ERR_UNSUPPORTED) return std::nullopt;
     check(rc, where);
     return out;
+}
+
+// Prefill MLP input over affine-Q4 gate and up matrices (an MoE layer's shared
+// expert): x [..., hidden] -> h [..., ffn] = fp16(fp16(silu(gate x)) * (up x)) on
+// the MFMA dequant-GEMM; None for shapes, groupings or alignments it does not serve.
+std::optional<torch::Tensor> fused_affine_gate_up_silu_gemm(torch::Tensor x, std::vector<AffineEntry> entries) {
+    const char* where = "fused_affine_gate_up_silu_gemm";
+    if (entries.size() != 2) throw std::runtime_error(std::string(where) + ": expects gate, up");
+    const gdsllm_affine_experts g = experts_of(entries[0], where), u = experts_of(entries[1], where);
+    const int dev = std::get<0>(entries[0])->device_id();
+    if (std::get<0>(entries[1])->device_id() != dev)
+        throw std::runtime_error(std::string(where) + ": buffers on different devices");
+    if (g.num_experts != 1 || u.num_experts != 1 || g.out_dim != u.out_dim || g.in_dim != u.in_dim ||
+        g.group_size != u.group_size)
+        return std::nullopt;
+    torch::Tensor xf = x.contiguous();
+    check_x(xf, dev, where);
+    if (g.in_dim <= 0 || xf.size(-1) != g.in_dim)
+        throw std::runtime_error(std::string(where) + ": last dim of x must equal in_dim " + std::to_string(g.in_dim));
+    const int64_t tokens = xf.numel() / g.in_dim;
+    auto out_shape = xf.sizes().vec();
+    out_shape.back() = g.out_dim;
+    torch::Tensor h = torch::empty(out_shape, fp16_on(dev));
+    torch::Tensor ws = gemm_workspace(g.out_dim, g.in_dim, tokens, dev, true);
+    const int rc = gdsllm_dequant_gemm_gate_up_silu_affine_q4(
+        g.weight, g.scales, g.biases, u.weight, u.scales, u.biases, xf.data_ptr(), h.data_ptr(), g.out_dim, g.in_dim,
+        g.group_size, tokens, g.in_dim, g.out_dim, ws.defined() ? ws.data_ptr() : nullptr,
+        ws.defined() ? ws.numel() : 0, OnDevice(dev).stream());
+    if (rc == GDSLLM_ERR_UNSUPPORTED) return std::nullopt;
+    check(rc, where);
+    return h;
 }
 
 // Prefill routed-expert MLP over resident stacked experts (the prefill branch
@@ -919,6 +952,9 @@ PYBIND11_MODULE(gds_io_ext, m) {
     m.def("moe_prefill_affine_q4", &moe_prefill_affine_q4,
           "Prefill routed-expert MLP over stacked experts: x [T, H] -> expert_output [T, H] (None if not served).",
           py::arg("x"), py::arg("entries"), py::arg("top_k_indices"), py::arg("top_k_weights"));
+    m.def("fused_affine_gate_up_silu_gemm", &fused_affine_gate_up_silu_gemm,
+          "Prefill affine-Q4 gate/up/SiLU on MFMA: x [T, K] -> h [T, F] (None if not served).", py::arg("x"),
+          py::arg("entries"));
     m.def("fused_gate_up_silu_gemm", &fused_gate_up_silu_gemm,
           "Prefill fp16(silu(gate . x) * (up . x)) on MFMA: x [..., K] -> h [..., M] (None if not served).",
           py::arg("gate_handle"), py::arg("up_handle"), py::arg("x"), py::arg("weight_shape"), py::arg("gguf_type"),

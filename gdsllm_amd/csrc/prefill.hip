@@ -6,7 +6,7 @@
 // (runtime/llama.py:160-166 for GGUF Q4_0 / Q8_0, runtime/qwen_moe.py:72-73
 // for affine-Q4), fused so the fp16 weight matrix never goes back to HBM.
 //
-// One split-K workgroup kernel serves three weight formats and five modes.
+// One split-K workgroup kernel serves three weight formats and six modes.
 //
 // Workgroup: 128 weight rows x BT tokens (BT = 64 or 32), 8 waves (two per
 // SIMD).  A stage is 128 values of k (four 32-value blocks); wave w takes
@@ -54,8 +54,8 @@
 //             0..BM/2-1 from the gate matrix and BM/2..BM-1 from the up matrix
 //             at the same BM/2 output rows, h written instead of g and u (the
 //             prefill form of the decode gate_up_silu, runtime/llama.py:253-256).
-//  * kDenseSplit  kDense over one of several parts of K, with fp32 partial sums
-//             stored instead of Y (split_sum adds them in part order): for
+//  * kDenseSplit, kDualSplit  kDense / kDenseDual over one of several parts of K, with fp32 partial sums
+//             stored instead of Y or h (split_sum adds them in part order): for
 //             launches whose tiles leave most compute units idle.
 //  * kDualSilu  kGather with rows 0..63 of the workgroup taken from the gate
 //             pool and rows 64..127 from the up pool at the same 64 output
@@ -71,7 +71,7 @@ namespace gdsllm {
 namespace {
 
 enum class WF { Q4_0, Q8_0, AFF32, AFF64, AFF128 };
-enum Mode { kDense = 0, kGather = 1, kDualSilu = 2, kDenseDual = 3, kDenseSplit = 4 };
+enum Mode { kDense = 0, kGather = 1, kDualSilu = 2, kDenseDual = 3, kDenseSplit = 4, kDualSplit = 5 };
 
 constexpr int kWaves = 8;
 constexpr int kBM = 128;     // weight rows per workgroup (or 256: the dense tile of gemm_sk)
@@ -162,9 +162,9 @@ struct GemmArgs {
     const int4* tiles;  // gather modes: (expert, p0, n, 0)
     const int* ntiles;
     const int* tok;     // gather modes: X row of each position
-    float* part;        // split mode: fp32 partial sums [ksplit][T][ldp]
+    float* part;        // split modes: fp32 partial sums [ksplit][T][ldp] (dual: [ksplit][gate, up][T][ldp])
     int64_t ldp;
-    int ksplit, ttiles; // split mode: parts of K, token tiles
+    int ksplit, ttiles; // split modes: parts of K, token tiles
 };
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
@@ -185,7 +185,8 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
     constexpr int SPS = Fm::SPS, XR = R::XR, RW = R::RW, CW = Fm::kCW;
     constexpr int kXSlot = R::kXSlot;
     constexpr bool kGath = MODE == kGather || MODE == kDualSilu;
-    constexpr bool kDual = MODE == kDualSilu || MODE == kDenseDual;
+    constexpr bool kDual = MODE == kDualSilu || MODE == kDenseDual || MODE == kDualSplit;
+    constexpr bool kSplit = MODE == kDenseSplit || MODE == kDualSplit;
     static_assert(MODE != kDualSilu || Fm::kAff, "the gathered dual tiles are built for the affine pools");
     static_assert(BM == kBM || MODE == kDense || MODE == kDenseDual, "the 256-row tile serves the dense modes only");
     constexpr int KS = kWaves * 64 / BM;  // waves along K (4 or 2)
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
 
     // ---- tile
     int m0, t0 = 0, nt, p0 = 0, nst = a.K / kStageK, split = 0;
-    int64_t k0 = 0;  // first k of this workgroup's part (split mode)
+    int64_t k0 = 0;  // first k of this workgroup's part (split modes)
     const uint8_t *wA = a.w, *sA = a.s, *bA = a.b, *wB = a.w2, *sB = a.s2, *bB = a.b2;
     if constexpr (kGath) {
         // The grid covers the worst case; the first ntiles * mtiles
@@ -233,7 +234,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
         const int q = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
         m0 = (q % a.mtiles) * (kDual ? BM / 2 : BM);
         int tt = q / a.mtiles;
-        if constexpr (MODE == kDenseSplit) {
+        if constexpr (kSplit) {
             // part `split` of K: whole units of 256 k, so every row's slot
             // windows start as they do at k = 0 (Q8_0's alternate by stage)
             split = tt / a.ttiles;
@@ -243,10 +244,18 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
             const int u1 = static_cast<int>(static_cast<int64_t>(units) * (split + 1) / a.ksplit);
             nst = 2 * (u1 - u0);
             k0 = 256 * static_cast<int64_t>(u0);
-            wA += Fm::kAff ? k0 / 2 : k0 / 32 * (F == WF::Q8_0 ? 34 : 18);
+            const int64_t ow = Fm::kAff ? k0 / 2 : k0 / 32 * (F == WF::Q8_0 ? 34 : 18), os = k0 / Fm::G * 2;
+            wA += ow;
             if constexpr (Fm::kAff) {
-                sA += k0 / Fm::G * 2;
-                bA += k0 / Fm::G * 2;
+                sA += os;
+                bA += os;
+            }
+            if constexpr (kDual) {
+                wB += ow;
+                if constexpr (Fm::kAff) {
+                    sB += os;
+                    bB += os;
+                }
             }
         }
         t0 = tt * BT;
@@ -659,7 +668,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
                         float4_t{av[4 * j], av[4 * j + 1], av[4 * j + 2], av[4 * j + 3]};
                 }
         __syncthreads();
-        if constexpr (!kDual) {
+        if constexpr (!kDual || kSplit) {
             // wave (kq, rq) stores units v = UPW*kq .. +UPW-1 of row block rq
             constexpr int UPW = 8 * PF / KS;
 #pragma unroll
@@ -667,12 +676,14 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
                 const int v = UPW * kq + z;
                 const int j = v & 3, fr = (v >> 2) & 1, f = v >> 3;
                 const float4_t sum = ksum(KS * rq, f, fr, j);
-                const int m = m0 + 64 * rq + 32 * fr + l32;
+                // dual: row block 0 is gate, 1 is up, at the same 64 rows
+                const int m = m0 + (kDual ? 0 : 64 * rq) + 32 * fr + l32;
+                const int plane = kDual ? 2 * split + rq : split;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int t = 32 * (pass * PF + f) + 8 * j + 4 * h + i;
-                    if constexpr (MODE == kDenseSplit) {
-                        if (t < nt && m < M) a.part[(static_cast<int64_t>(split) * a.T + t0 + t) * a.ldp + m] = sum[i];
+                    if constexpr (kSplit) {
+                        if (t < nt && m < M) a.part[(static_cast<int64_t>(plane) * a.T + t0 + t) * a.ldp + m] = sum[i];
                     } else {
                         if (t < nt && m < M) a.y[yrow(t) * a.ldy + m] = f2h_bits(sum[i]);
                     }
@@ -752,27 +763,39 @@ inline Tile pick_tile(int64_t rows, int64_t T, int64_t K, bool allow256) {
     return c128 < c64 ? Tile::k128x128 : Tile::k128x64;
 }
 
-// y[t][m..m+3] = fp16 of the K parts' partial sums, added in part order.
-template <bool VEC>
+// y[t][m..m+3] = fp16 of the K parts' partial sums, added in part order; DUAL:
+// h = fp16(fp16(silu(g)) * u) of the gate and up sums, as kDenseDual writes it.
+template <bool VEC, bool DUAL>
 __global__ __launch_bounds__(256) void split_sum(const float* __restrict__ part, int64_t ldp, int ksplit, int M, int T,
                                                  uint16_t* __restrict__ y, int64_t ldy) {
     const int64_t q = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, per = ldp / 4;
     if (q >= per * T) return;
     const int64_t t = q / per, m = 4 * (q % per), plane = static_cast<int64_t>(T) * ldp;
     const float* p = part + t * ldp + m;
-    float4_t sum = *reinterpret_cast<const float4_t*>(p);
+    auto total = [&](const float* p0) {
+        float4_t sum = *reinterpret_cast<const float4_t*>(p0);
 #pragma unroll 4
-    for (int s = 1; s < ksplit; ++s) sum += *reinterpret_cast<const float4_t*>(p + s * plane);
+        for (int s = 1; s < ksplit; ++s) sum += *reinterpret_cast<const float4_t*>(p0 + (DUAL ? 2 * s : s) * plane);
+        return sum;
+    };
+    const float4_t sum = total(p);
+    uint16_t v[4];
+    if constexpr (DUAL) {
+        const float4_t up = total(p + plane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = silu_mul_h(sum[i], up[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = f2h_bits(sum[i]);
+    }
     uint16_t* o = y + t * ldy + m;
     if constexpr (VEC) {
-        uint2 v;
-        v.x = f2h_bits(sum[0]) | (static_cast<uint32_t>(f2h_bits(sum[1])) << 16);
-        v.y = f2h_bits(sum[2]) | (static_cast<uint32_t>(f2h_bits(sum[3])) << 16);
-        *reinterpret_cast<uint2*>(o) = v;
+        *reinterpret_cast<uint2*>(o) = make_uint2(v[0] | (static_cast<uint32_t>(v[1]) << 16),
+                                                  v[2] | (static_cast<uint32_t>(v[3]) << 16));
     } else {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            if (m + i < M) o[i] = f2h_bits(sum[i]);
+            if (m + i < M) o[i] = v[i];
     }
 }
 
@@ -795,9 +818,10 @@ struct SplitPlan {
     int bt = 0, parts = 1;
 };
 inline int64_t split_ld(int64_t M) { return (M + 3) / 4 * 4; }
-inline size_t split_bytes(const SplitPlan& p, int64_t M, int64_t T) {
-    return p.parts > 1 ? static_cast<size_t>(p.parts) * T * split_ld(M) * sizeof(float) : 0;
+inline size_t split_bytes(const SplitPlan& p, int64_t M, int64_t T, bool dual) {
+    return p.parts > 1 ? static_cast<size_t>(p.parts) * (dual ? 2 : 1) * T * split_ld(M) * sizeof(float) : 0;
 }
+// M: the rows of a launch's tiles (gate/up/SiLU: gate and up rows together).
 inline SplitPlan pick_split(int64_t M, int64_t T, int64_t K) {
     const int64_t cu = cu_count(), units = K / 256;
     if (M <= 0 || T <= 0 || K % 256 != 0) return {};
@@ -821,34 +845,40 @@ inline SplitPlan pick_split(int64_t M, int64_t T, int64_t K) {
     return best;
 }
 
-template <WF F, int BT>
-int dense_split_gemm(GemmArgs a, const SplitPlan& p, float* part, hipStream_t stream) {
-    a.mtiles = (a.M + kBM - 1) / kBM;
+template <WF F, int BT, bool DUAL>
+int split_gemm(GemmArgs a, const SplitPlan& p, float* part, hipStream_t stream) {
+    a.mtiles = DUAL ? (a.M + kBM / 2 - 1) / (kBM / 2) : (a.M + kBM - 1) / kBM;
     a.ttiles = (a.T + BT - 1) / BT;
     a.ksplit = p.parts;
     a.part = part;
     a.ldp = split_ld(a.M);
     // pick_split splits only launches of few tiles, so the grid stays small
-    if (int rc = launch_sk<F, BT, kDenseSplit>(a, static_cast<unsigned>(a.mtiles) * a.ttiles * a.ksplit, stream)) return rc;
+    const unsigned nwg = static_cast<unsigned>(a.mtiles) * a.ttiles * a.ksplit;
+    if (int rc = launch_sk<F, BT, DUAL ? kDualSplit : kDenseSplit>(a, nwg, stream)) return rc;
     const int64_t threads = a.ldp / 4 * a.T;
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
     if (a.M % 4 == 0 && a.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(a.y) % 8 == 0)
-        hipLaunchKernelGGL((split_sum<true>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
+        hipLaunchKernelGGL((split_sum<true, DUAL>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
     else
-        hipLaunchKernelGGL((split_sum<false>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
+        hipLaunchKernelGGL((split_sum<false, DUAL>), grid, dim3(256), 0, stream, part, a.ldp, a.ksplit, a.M, a.T, a.y, a.ldy);
     return check_hip(hipGetLastError(), "split_sum launch");
+}
+
+// The split launch where the plan has one and the workspace holds it, else -1.
+template <WF F, bool DUAL>
+int try_split(const GemmArgs& a, void* workspace, size_t bytes, hipStream_t stream) {
+    if (!workspace) return -1;
+    const SplitPlan p = pick_split(DUAL ? 2 * static_cast<int64_t>(a.M) : a.M, a.T, a.K);
+    const size_t need = split_bytes(p, a.M, a.T, DUAL);
+    if (need == 0 || need > bytes) return -1;
+    float* part = static_cast<float*>(workspace);
+    return p.bt == 128 ? split_gemm<F, 128, DUAL>(a, p, part, stream) : split_gemm<F, 64, DUAL>(a, p, part, stream);
 }
 
 template <WF F>
 int dense_gemm_auto(const GemmArgs& a, void* workspace, size_t bytes, hipStream_t stream) {
-    if (workspace) {
-        const SplitPlan p = pick_split(a.M, a.T, a.K);
-        const size_t need = split_bytes(p, a.M, a.T);
-        if (need > 0 && need <= bytes) {
-            float* part = static_cast<float*>(workspace);
-            return p.bt == 128 ? dense_split_gemm<F, 128>(a, p, part, stream) : dense_split_gemm<F, 64>(a, p, part, stream);
-        }
-    }
+    const int rc = try_split<F, false>(a, workspace, bytes, stream);
+    if (rc != -1) return rc;
     switch (pick_tile(a.M, a.T, a.K, true)) {
         case Tile::k256x128: return dense_gemm<F, 128, 2 * kBM>(a, stream);
         case Tile::k128x128: return dense_gemm<F, 128>(a, stream);
@@ -883,7 +913,9 @@ int dense_dual_gemm(GemmArgs a, hipStream_t stream) {
 // launch at 512 tokens, 2 rounds against 3, measured 138.9 against 134.8 us
 // with 128-row tiles); affine weights keep 128-row tiles.
 template <WF F>
-int dense_dual_gemm_auto(const GemmArgs& a, hipStream_t stream) {
+int dense_dual_gemm_auto(const GemmArgs& a, void* workspace, size_t bytes, hipStream_t stream) {
+    const int rc = try_split<F, true>(a, workspace, bytes, stream);
+    if (rc != -1) return rc;
     const int64_t rows = 2 * static_cast<int64_t>(a.M), cu = cu_count();
     const int64_t r128 = ((rows + 127) / 128 * ((a.T + 127) / 128) + cu - 1) / cu;
     const int64_t r256 = ((rows + 255) / 256 * ((a.T + 127) / 128) + cu - 1) / cu;
@@ -1215,7 +1247,11 @@ int run_dense(const void* w, const void* s, const void* b, const void* x, void* 
 }  // namespace
 
 extern "C" size_t gdsllm_dequant_gemm_workspace_size(int64_t out_dim, int64_t in_dim, int64_t tokens) {
-    return split_bytes(pick_split(out_dim, tokens, in_dim), out_dim, tokens);
+    return split_bytes(pick_split(out_dim, tokens, in_dim), out_dim, tokens, false);
+}
+
+extern "C" size_t gdsllm_dequant_gemm_gate_up_silu_workspace_size(int64_t ffn_dim, int64_t in_dim, int64_t tokens) {
+    return split_bytes(pick_split(2 * ffn_dim, tokens, in_dim), ffn_dim, tokens, true);
 }
 
 extern "C" int gdsllm_dequant_gemm_q8_0_ws(const void* weight, const void* x, void* y, int64_t out_dim, int64_t in_dim,
@@ -1359,8 +1395,32 @@ extern "C" int gdsllm_moe_prefill_affine_q4(const gdsllm_affine_experts* gate, c
 
 namespace {
 template <WF F>
+int run_dual(const void* const (&g)[3], const void* const (&u)[3], const void* x, void* h, int64_t M, int64_t K,
+             int64_t T, int64_t ldx, int64_t ldh, void* workspace, size_t bytes, void* stream) {
+    if (reinterpret_cast<uintptr_t>(workspace) % 16)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, "dequant_gemm_gate_up_silu: workspace must be 16-byte aligned");
+    GemmArgs a{};
+    a.w = static_cast<const uint8_t*>(g[0]);
+    a.s = static_cast<const uint8_t*>(g[1]);
+    a.b = static_cast<const uint8_t*>(g[2]);
+    a.w2 = static_cast<const uint8_t*>(u[0]);
+    a.s2 = static_cast<const uint8_t*>(u[1]);
+    a.b2 = static_cast<const uint8_t*>(u[2]);
+    a.x = static_cast<const uint16_t*>(x);
+    a.y = static_cast<uint16_t*>(h);
+    a.M = static_cast<int>(M);
+    a.K = static_cast<int>(K);
+    a.T = static_cast<int>(T);
+    a.ldx = ldx;
+    a.ldy = ldh;
+    const int rc = dense_dual_gemm_auto<F>(a, workspace, bytes, as_stream(stream));
+    return rc == GDSLLM_OK ? ok() : rc;
+}
+
+template <WF F>
 int gate_up_silu_entry(const std::string& n, const void* gate, const void* up, const void* x, void* h,
-                       int64_t ffn_dim, int64_t in_dim, int64_t tokens, int64_t ldx, int64_t ldh, void* stream) {
+                       int64_t ffn_dim, int64_t in_dim, int64_t tokens, int64_t ldx, int64_t ldh, void* workspace,
+                       size_t workspace_bytes, void* stream) {
     bool empty;
     if (int rc = check_dense(n, gate, x, h, ffn_dim, in_dim, tokens, ldx, ldh, empty)) return rc;
     if (empty) return ok();
@@ -1370,31 +1430,71 @@ int gate_up_silu_entry(const std::string& n, const void* gate, const void* up, c
     if (in_dim % 256 != 0) return off_grid(n, in_dim);
     if (F == WF::Q8_0)
         if (int rc = check_q8_rows(n, in_dim)) return rc;
-    GemmArgs a{};
-    a.w = static_cast<const uint8_t*>(gate);
-    a.w2 = static_cast<const uint8_t*>(up);
-    a.x = static_cast<const uint16_t*>(x);
-    a.y = static_cast<uint16_t*>(h);
-    a.M = static_cast<int>(ffn_dim);
-    a.K = static_cast<int>(in_dim);
-    a.T = static_cast<int>(tokens);
-    a.ldx = ldx;
-    a.ldy = ldh;
-    const int rc = dense_dual_gemm_auto<F>(a, as_stream(stream));
-    return rc == GDSLLM_OK ? ok() : rc;
+    return run_dual<F>({gate, nullptr, nullptr}, {up, nullptr, nullptr}, x, h, ffn_dim, in_dim, tokens, ldx, ldh,
+                       workspace, workspace_bytes, stream);
 }
 }  // namespace
+
+extern "C" int gdsllm_dequant_gemm_gate_up_silu_q4_0_ws(const void* gate_weight, const void* up_weight, const void* x,
+                                                        void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
+                                                        int64_t ldx, int64_t ldh, void* workspace,
+                                                        size_t workspace_bytes, void* stream) {
+    return gate_up_silu_entry<WF::Q4_0>("dequant_gemm_gate_up_silu_q4_0", gate_weight, up_weight, x, h, ffn_dim,
+                                        in_dim, tokens, ldx, ldh, workspace, workspace_bytes, stream);
+}
+
+extern "C" int gdsllm_dequant_gemm_gate_up_silu_q8_0_ws(const void* gate_weight, const void* up_weight, const void* x,
+                                                        void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
+                                                        int64_t ldx, int64_t ldh, void* workspace,
+                                                        size_t workspace_bytes, void* stream) {
+    return gate_up_silu_entry<WF::Q8_0>("dequant_gemm_gate_up_silu_q8_0", gate_weight, up_weight, x, h, ffn_dim,
+                                        in_dim, tokens, ldx, ldh, workspace, workspace_bytes, stream);
+}
 
 extern "C" int gdsllm_dequant_gemm_gate_up_silu_q4_0(const void* gate_weight, const void* up_weight, const void* x,
                                                      void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
                                                      int64_t ldx, int64_t ldh, void* stream) {
-    return gate_up_silu_entry<WF::Q4_0>("dequant_gemm_gate_up_silu_q4_0", gate_weight, up_weight, x, h, ffn_dim,
-                                        in_dim, tokens, ldx, ldh, stream);
+    return gdsllm_dequant_gemm_gate_up_silu_q4_0_ws(gate_weight, up_weight, x, h, ffn_dim, in_dim, tokens, ldx, ldh,
+                                                    nullptr, 0, stream);
 }
 
 extern "C" int gdsllm_dequant_gemm_gate_up_silu_q8_0(const void* gate_weight, const void* up_weight, const void* x,
                                                      void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
                                                      int64_t ldx, int64_t ldh, void* stream) {
-    return gate_up_silu_entry<WF::Q8_0>("dequant_gemm_gate_up_silu_q8_0", gate_weight, up_weight, x, h, ffn_dim,
-                                        in_dim, tokens, ldx, ldh, stream);
+    return gdsllm_dequant_gemm_gate_up_silu_q8_0_ws(gate_weight, up_weight, x, h, ffn_dim, in_dim, tokens, ldx, ldh,
+                                                    nullptr, 0, stream);
+}
+
+extern "C" int gdsllm_dequant_gemm_gate_up_silu_affine_q4(const void* gate_weight, const void* gate_scales,
+                                                          const void* gate_biases, const void* up_weight,
+                                                          const void* up_scales, const void* up_biases, const void* x,
+                                                          void* h, int64_t ffn_dim, int64_t in_dim, int64_t group_size,
+                                                          int64_t tokens, int64_t ldx, int64_t ldh, void* workspace,
+                                                          size_t workspace_bytes, void* stream) {
+    const std::string n = "dequant_gemm_gate_up_silu_affine_q4";
+    if (group_size <= 0 || group_size % 8 != 0)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": group_size must be a positive multiple of 8");
+    bool empty;
+    if (int rc = check_dense(n, gate_weight, x, h, ffn_dim, in_dim, tokens, ldx, ldh, empty)) return rc;
+    if (empty) return ok();
+    if (in_dim % group_size != 0)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": in_dim must be a multiple of group_size");
+    if (!gate_scales || !gate_biases || !up_weight || !up_scales || !up_biases)
+        return set_error(GDSLLM_ERR_INVALID_ARGUMENT, n + ": null pointer");
+    if (in_dim % 256 != 0) return off_grid(n, in_dim);
+    if (group_size != 32 && group_size != 64 && group_size != 128)
+        return set_error(GDSLLM_ERR_UNSUPPORTED, n + ": the MFMA GEMM takes group_size 32, 64 or 128");
+    const uintptr_t sal = group_size == 32 ? 16 : 4;
+    for (const void* p : {gate_scales, gate_biases, up_scales, up_biases})
+        if (reinterpret_cast<uintptr_t>(p) % sal)
+            return set_error(GDSLLM_ERR_UNSUPPORTED, n + ": scales/biases must be " + std::to_string(sal) + "-byte aligned");
+    if (reinterpret_cast<uintptr_t>(up_weight) % 16)
+        return set_error(GDSLLM_ERR_UNSUPPORTED, n + ": weight and x rows must be 16-byte aligned (ldx % 8 == 0)");
+    const void* const g[3] = {gate_weight, gate_scales, gate_biases};
+    const void* const u[3] = {up_weight, up_scales, up_biases};
+    switch (group_size) {
+        case 32: return run_dual<WF::AFF32>(g, u, x, h, ffn_dim, in_dim, tokens, ldx, ldh, workspace, workspace_bytes, stream);
+        case 64: return run_dual<WF::AFF64>(g, u, x, h, ffn_dim, in_dim, tokens, ldx, ldh, workspace, workspace_bytes, stream);
+        default: return run_dual<WF::AFF128>(g, u, x, h, ffn_dim, in_dim, tokens, ldx, ldh, workspace, workspace_bytes, stream);
+    }
 }

@@ -23,7 +23,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ext
-from .llama import prefill_takes_fused_gemm
+from .llama import FUSED_GEMM_MAX_TOKENS, prefill_takes_fused_gemm
 
 
 def _dequant_affine_q4(meta: dict, scratch: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -134,6 +134,24 @@ def _entry(m: dict) -> tuple:
     return (m["buffer"], list(m["shape"]), m["weight_offset"], m["scale_offset"], m["bias_offset"], m["group_size"])
 
 
+def _shared_gate_up_silu(x: torch.Tensor, weights: Dict) -> Optional[torch.Tensor]:
+    """h = silu(gate x) * (up x) of the shared expert of a prefill chunk
+    (runtime/qwen_moe.py:497-505) in one MFMA launch, split along K where its
+    tiles are few (512 tokens over 1024 x 4096: 29 us, against 60 us as two
+    dequants, two GEMMs and the elementwise ops).  Long chunks over many rows
+    keep the separate route, which dequantizes once per call (the line of
+    prefill_takes_fused_gemm).  None where the launch does not apply."""
+    g, u = (weights.get(f"{p}.weight") for p in _SHARED_PROJ[:2])
+    if not all(isinstance(m, dict) and m.get("quant_type") == "affine_q4" and len(m["shape"]) == 2 for m in (g, u)):
+        return None
+    if list(g["shape"]) != list(u["shape"]) or g["group_size"] != u["group_size"] or \
+            g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8):
+        return None
+    if x.numel() // x.shape[-1] > FUSED_GEMM_MAX_TOKENS and 2 * int(g["shape"][0]) > 8192:
+        return None
+    return ext().fused_affine_gate_up_silu_gemm(x, [_entry(g), _entry(u)])
+
+
 def moe_step(x: torch.Tensor, weights: Dict, top_k_indices: torch.Tensor, top_k_weights: torch.Tensor):
     """The decode MoE MLP of runtime/qwen_moe.py:455-513 for one token in two
     launches: one for the gate/up rows of the top-k experts and the shared
@@ -228,9 +246,12 @@ def moe_mlp_selective(
 
     if "mlp.shared_expert.gate_proj.weight" not in weights:
         return expert_output.clamp(min=-65504.0, max=65504.0)
-    shared_gate = affine_q4_linear(x, weights, "mlp.shared_expert.gate_proj", scratch)
-    shared_up = affine_q4_linear(x, weights, "mlp.shared_expert.up_proj", scratch)
-    shared_out = affine_q4_linear(F.silu(shared_gate) * shared_up, weights, "mlp.shared_expert.down_proj", scratch)
+    shared_h = _shared_gate_up_silu(x, weights)
+    if shared_h is None:
+        shared_gate = affine_q4_linear(x, weights, "mlp.shared_expert.gate_proj", scratch)
+        shared_up = affine_q4_linear(x, weights, "mlp.shared_expert.up_proj", scratch)
+        shared_h = F.silu(shared_gate) * shared_up
+    shared_out = affine_q4_linear(shared_h, weights, "mlp.shared_expert.down_proj", scratch)
     sg = weights["mlp.shared_expert_gate.weight"]
     if isinstance(sg, dict):
         gate_logit = affine_q4_linear(x, weights, "mlp.shared_expert_gate", scratch)

@@ -136,8 +136,8 @@ int gdsllm_fused_int8_gemv(const void* weight, const void* scale, const void* x,
  * compute unit a workgroup, with in_dim over 2-4 windows of 4096, adds its
  * window sums in another order, and for Q4_0 at batch 3-8, where the group
  * launch sums the same block products in the x-in-registers kernel's order:
- * equal to fp32 rounding); shapes no single-launch kernel serves (batch 3-8
- * Q8_0, in_dim > 8192 or not a multiple of 256 at batch 3-8, unaligned
+ * equal to fp32 rounding); shapes no single-launch kernel serves (in_dim >
+ * 8192 or not a multiple of 256 at batch 3-8, unaligned
  * weights or x) fall back to one launch per matrix.                          */
 int gdsllm_fused_q4_0_gemv_group(int n, const void* const* weights, void* const* ys,
                                  const int64_t* out_dims, const void* x, int64_t in_dim,
@@ -362,6 +362,25 @@ int gdsllm_dequant_gemm_gate_up_silu_q4_0(const void* gate_weight, const void* u
 int gdsllm_dequant_gemm_gate_up_silu_q8_0(const void* gate_weight, const void* up_weight, const void* x,
                                           void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
                                           int64_t ldx, int64_t ldh, void* stream);
+/* The same with a device workspace, split along K as
+ * gdsllm_dequant_gemm_*_ws split theirs, and on affine-Q4 matrices (the shared
+ * expert of an MoE prefill chunk; the limits of gdsllm_dequant_gemm_affine_q4,
+ * workspace null where K is not to be split).                              */
+size_t gdsllm_dequant_gemm_gate_up_silu_workspace_size(int64_t ffn_dim, int64_t in_dim, int64_t tokens);
+int gdsllm_dequant_gemm_gate_up_silu_q4_0_ws(const void* gate_weight, const void* up_weight, const void* x,
+                                             void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
+                                             int64_t ldx, int64_t ldh, void* workspace,
+                                             size_t workspace_bytes, void* stream);
+int gdsllm_dequant_gemm_gate_up_silu_q8_0_ws(const void* gate_weight, const void* up_weight, const void* x,
+                                             void* h, int64_t ffn_dim, int64_t in_dim, int64_t tokens,
+                                             int64_t ldx, int64_t ldh, void* workspace,
+                                             size_t workspace_bytes, void* stream);
+int gdsllm_dequant_gemm_gate_up_silu_affine_q4(const void* gate_weight, const void* gate_scales,
+                                               const void* gate_biases, const void* up_weight,
+                                               const void* up_scales, const void* up_biases, const void* x,
+                                               void* h, int64_t ffn_dim, int64_t in_dim, int64_t group_size,
+                                               int64_t tokens, int64_t ldx, int64_t ldh, void* workspace,
+                                               size_t workspace_bytes, void* stream);
 
 /* Bytes of device workspace gdsllm_moe_prefill_affine_q4 needs. */
 size_t gdsllm_moe_prefill_workspace_size(int64_t tokens, int64_t top_k, int64_t ffn_dim,

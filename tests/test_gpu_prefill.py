@@ -512,3 +512,57 @@ def test_dequant_gemm_split_k(gpu, fmt, T, M, K):
     a, b = a.astype(np.float64), b.astype(np.float64)
     bound = oq.fp16_ulp(np.maximum(np.abs(a), np.abs(b))) + oq.row_norms(deq, to_np(x)) * 2.0 ** -16
     assert (np.abs(a - b) <= bound).all()
+
+
+# (T, F, K) of the gate/up/SiLU launch split along K: equal and unequal parts,
+# ffn rows off the 64 grid and off the 4-row vector store, ragged token tiles;
+# the last does not split.
+SPLIT_DUAL_CASES = [(9, 512, 2048), (37, 389, 5888), (100, 1026, 4096), (512, 1024, 4096), (512, 11008, 256)]
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "affine32", "affine64", "affine128"])
+@pytest.mark.parametrize("T,F,K", SPLIT_DUAL_CASES, ids=[f"T{t}_{m}x{k}" for t, m, k in SPLIT_DUAL_CASES])
+def test_dequant_gemm_gate_up_silu_split_k(gpu, fmt, T, F, K):
+    """h of the split launch and of the whole-K one (no workspace) end to end
+    against the oracle's g and u (relative L2); the two within what fp32
+    reassociation of g and u allows, as in test_dequant_gemm_gate_up_silu;
+    bytes past the workspace and columns past the rows stay as they were."""
+    x = syn.activations(T, K, gen(5901 + T))
+    xd, ldh = x.to(gpu), F + 3
+    need = capi().gdsllm_dequant_gemm_gate_up_silu_workspace_size(F, K, T)
+    assert (need > 0) == (F < 11008)
+    ws = torch.full((need + 256,), 0xA5, dtype=torch.uint8, device=gpu)
+    hs = [torch.full((T, ldh), 7.0, dtype=torch.float16, device=gpu) for _ in range(2)]
+    if fmt.startswith("affine"):
+        g = int(fmt[6:])
+        raw = [syn.affine_q4_weights([F, K], g, gen(5902 + i)) for i in range(2)]
+        deqs = [affine_dequant_np(*r, g).reshape(F, K) for r in raw]
+        dev = [t.to(gpu) for r in raw for t in r]
+
+        def run(h, wp, nb):
+            return capi().gdsllm_dequant_gemm_gate_up_silu_affine_q4(*[ptr(t) for t in dev], ptr(xd), ptr(h), F, K, g, T,
+                                                                     K, ldh, wp, nb, stream())
+    else:
+        raw = [(syn.q4_0_weights if fmt == "q4_0" else syn.q8_0_weights)(F, K, gen(5902 + i)) for i in range(2)]
+        deqs = [(oq.dequant_q4_0 if fmt == "q4_0" else oq.dequant_q8_0)(to_np(r)).reshape(F, K) for r in raw]
+        dev = [r.to(gpu) for r in raw]
+        fn = (capi().gdsllm_dequant_gemm_gate_up_silu_q4_0_ws if fmt == "q4_0"
+              else capi().gdsllm_dequant_gemm_gate_up_silu_q8_0_ws)
+
+        def run(h, wp, nb):
+            return fn(ptr(dev[0]), ptr(dev[1]), ptr(xd), ptr(h), F, K, T, K, ldh, wp, nb, stream())
+    check(run(hs[0], ptr(ws), need))
+    check(run(hs[1], None, 0))
+    torch.cuda.synchronize()
+    assert bool((ws[need:] == 0xA5).all()), "bytes past the workspace were written"
+    assert all((to_np(h)[:, F:] == 7.0).all() for h in hs), "columns past the rows were written"
+    gq, uq = (oq.gemv(d, to_np(x)).astype(np.float16) for d in deqs)
+    want = (oq.silu_fp16(gq).astype(np.float32) * uq.astype(np.float32)).astype(np.float64)
+    a, b = (to_np(h)[:, :F].astype(np.float64) for h in hs)
+    for got in (a, b):
+        rel = float(np.linalg.norm(got - want) / np.linalg.norm(want))
+        assert rel <= oq.GEMV_REL_L2, f"{fmt} h rel L2 {rel:.3e}"
+    eg, eu = (oq.fp16_ulp(v) + oq.row_norms(d, to_np(x)) * 2.0 ** -16 for v, d in ((gq, deqs[0]), (uq, deqs[1])))
+    sg = np.abs(oq.silu_fp16(gq).astype(np.float64))
+    bound = 2 * ((1.1 * eg + oq.fp16_ulp(sg)) * (np.abs(uq.astype(np.float64)) + eu) + sg * eu + oq.fp16_ulp(want))
+    assert (np.abs(a - b) <= bound).all()
