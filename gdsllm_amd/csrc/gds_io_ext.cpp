@@ -796,6 +796,19 @@ torch::Tensor moe_combine(torch::Tensor expert_out, torch::Tensor shared_out, to
     return y;
 }
 
+// silu(gate) * up with torch fp16 semantics in one launch (runtime/llama.py:253-256).
+torch::Tensor silu_mul(torch::Tensor gate, torch::Tensor up) {
+    const char* where = "silu_mul";
+    check_fp16_cuda(gate, "gate", where);
+    check_fp16_cuda(up, "up", where);
+    torch::Tensor g = gate.contiguous(), u = up.contiguous();
+    if (!g.sizes().equals(u.sizes()) || g.device() != u.device())
+        throw std::runtime_error(std::string(where) + ": gate and up differ in shape or device");
+    torch::Tensor h = torch::empty_like(g);
+    check(gdsllm_silu_mul(g.data_ptr(), u.data_ptr(), h.data_ptr(), g.numel(), OnDevice(g.get_device()).stream()), where);
+    return h;
+}
+
 // q/k/v-style projections sharing x in one launch (the decode step's
 // runtime/llama.py:212-214): one output [batch, out_dim_i] per matrix.
 std::vector<torch::Tensor> fused_dequant_gemv_group(const std::vector<Handle>& handles, torch::Tensor x,
@@ -969,6 +982,7 @@ PYBIND11_MODULE(gds_io_ext, m) {
           py::arg("weight"), py::arg("scale"), py::arg("x"));
     m.def("moe_route_topk", &moe_route_topk, "Top-k experts and fp16(softmax_fp32) weights from fp16 logits.",
           py::arg("logits"), py::arg("top_k"));
+    m.def("silu_mul", &silu_mul, "silu(gate) * up with torch fp16 semantics.", py::arg("gate"), py::arg("up"));
     m.def("moe_combine", &moe_combine, "clamp(expert_out + sigmoid(gate) * shared_out) with torch fp16 semantics.",
           py::arg("expert_out"), py::arg("shared_out"), py::arg("shared_gate_logit"));
 }

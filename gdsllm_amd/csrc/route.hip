@@ -176,6 +176,26 @@ __global__ __launch_bounds__(64) void route_topk(const uint16_t* __restrict__ lo
     topk_wave<NPL>(logits + t * ld, E, k, idx + t * k, wts + t * k, static_cast<int>(threadIdx.x));
 }
 
+// h = fp16(fp16(silu(g)) * u), 8 elements per thread (VEC: every pointer on the
+// 16-byte grid; the last thread takes the remainder one by one).  Bound by
+// memory: 2048 x 11008 is 135 MB, where torch's SiLU and product in two passes
+// move 225 MB (24.5 + 21.7 us); at decode size it saves a launch (2 x 4.6 us).
+template <bool VEC>
+__global__ __launch_bounds__(256) void silu_mul(const uint16_t* g, const uint16_t* u, uint16_t* h, int64_t n) {
+    const int64_t i0 = 8 * (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x);
+    if (i0 >= n) return;
+    if (VEC && i0 + 8 <= n) {
+        const uint4 gv = *reinterpret_cast<const uint4*>(g + i0), uv = *reinterpret_cast<const uint4*>(u + i0);
+        auto two = [](uint32_t a, uint32_t b) {
+            return static_cast<uint32_t>(silu_mul_h(h2f(a & 0xFFFFu), h2f(b & 0xFFFFu))) |
+                   (static_cast<uint32_t>(silu_mul_h(h2f(a >> 16), h2f(b >> 16))) << 16);
+        };
+        *reinterpret_cast<uint4*>(h + i0) = make_uint4(two(gv.x, uv.x), two(gv.y, uv.y), two(gv.z, uv.z), two(gv.w, uv.w));
+    } else {
+        for (int64_t i = i0; i < i0 + 8 && i < n; ++i) h[i] = silu_mul_h(h2f(g[i]), h2f(u[i]));
+    }
+}
+
 // y = clamp(e + fp16(fp16(sigmoid(g)) * s), -65504, 65504) elementwise, g per token.
 __global__ __launch_bounds__(256) void moe_combine(const uint16_t* __restrict__ eo, const uint16_t* __restrict__ so,
                                                    const uint16_t* __restrict__ gl, uint16_t* __restrict__ y,
@@ -328,5 +348,20 @@ extern "C" int gdsllm_moe_combine(const void* expert_out, const void* shared_out
                        static_cast<const uint16_t*>(expert_out), static_cast<const uint16_t*>(shared_out),
                        static_cast<const uint16_t*>(shared_gate_logit), static_cast<uint16_t*>(y), hidden, total);
     if (int rc = check_hip(hipGetLastError(), "moe_combine launch")) return rc;
+    return ok();
+}
+
+extern "C" int gdsllm_silu_mul(const void* gate, const void* up, void* h, int64_t n, void* stream) {
+    const std::string nm = "silu_mul";
+    if (n < 0 || n > (int64_t(1) << 40)) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, nm + ": n out of range");
+    if (n == 0) return ok();
+    if (!gate || !up || !h) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, nm + ": null pointer");
+    const uintptr_t bits = reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) | reinterpret_cast<uintptr_t>(h);
+    if (bits % 2) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, nm + ": pointers must be 2-byte aligned");
+    const dim3 grid(static_cast<unsigned>((n + 2047) / 2048));
+    const auto *g = static_cast<const uint16_t*>(gate), *u = static_cast<const uint16_t*>(up);
+    if (bits % 16 == 0) hipLaunchKernelGGL(silu_mul<true>, grid, dim3(256), 0, as_stream(stream), g, u, static_cast<uint16_t*>(h), n);
+    else hipLaunchKernelGGL(silu_mul<false>, grid, dim3(256), 0, as_stream(stream), g, u, static_cast<uint16_t*>(h), n);
+    if (int rc = check_hip(hipGetLastError(), "silu_mul launch")) return rc;
     return ok();
 }

@@ -137,6 +137,15 @@ def _gguf_pair(g, u) -> bool:
             g["buffer"].device_id == u["buffer"].device_id)
 
 
+def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """F.silu(gate) * up (runtime/llama.py:253-256): one launch for fp16 on the
+    device, torch's ops otherwise (and where gradients are recorded)."""
+    if (gate.is_cuda and gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape and
+            gate.device == up.device and not (gate.requires_grad or up.requires_grad)):
+        return ext().silu_mul(gate, up)
+    return F.silu(gate) * up
+
+
 def mlp(x: torch.Tensor, weights: Dict, scratch: Optional[torch.Tensor] = None) -> torch.Tensor:
     """SwiGLU MLP (runtime/llama.py:247-256).  Over GGUF weights h =
     fp16(silu(gate x) * (up x)) comes from one launch that never writes gate
@@ -158,4 +167,4 @@ def mlp(x: torch.Tensor, weights: Dict, scratch: Optional[torch.Tensor] = None) 
             return dequant_linear(h, weights, "mlp.down_proj", scratch)
     gate = dequant_linear(x, weights, "mlp.gate_proj", scratch)
     up = dequant_linear(x, weights, "mlp.up_proj", scratch)
-    return dequant_linear(F.silu(gate) * up, weights, "mlp.down_proj", scratch)
+    return dequant_linear(silu_mul(gate, up), weights, "mlp.down_proj", scratch)

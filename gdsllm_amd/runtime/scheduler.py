@@ -82,9 +82,10 @@ class DecodeSweep:
     the lm_head entry.  All weights one GGUF type; batch 1-8.  Where the
     fused gate/up/SiLU launch does not serve the shape (Q8_0 at batch 3-8, a
     hidden size it refuses) the layer's MLP input runs through the gate and
-    up GEMVs into scratch rows and h = silu(g) * u comes from torch's fp16
-    ops, the reference's own composition (runtime/llama.py:253-256): 5
-    launches per layer instead of 4, in the same graph.
+    up projections (one grouped launch into scratch rows) and h = silu(g) * u
+    in an elementwise launch, the reference's composition
+    (runtime/llama.py:253-256): 5 launches per layer instead of 4, in the
+    same graph.
     """
 
     def __init__(self, layers: Sequence[dict], lm_head: dict, batch: int = 1, device=None, use_graph: bool = True):
@@ -132,6 +133,8 @@ class DecodeSweep:
         self._qkv = [((c_vp * 3)(*[_ptr(m) for m in lm[:3]]),
                       (c_vp * 3)(self.q[i].data_ptr(), self.k[i].data_ptr(), self.v[i].data_ptr()),
                       (c_i64 * 3)(*[int(m["shape"][0]) for m in lm[:3]])) for i, lm in enumerate(metas)]
+        self._gate_up = [((c_vp * 2)(*[_ptr(m) for m in lm[4:6]]), (c_vp * 2)(self._g.data_ptr(), self._u.data_ptr()),
+                          (c_i64 * 2)(Fd, Fd)) for lm in metas]
         self._graph = None
 
     def _launch_all(self) -> None:
@@ -150,12 +153,12 @@ class DecodeSweep:
             check(gemv(_ptr(lm[3]), self.attn_out[i].data_ptr(), self.o[i].data_ptr(), mo, ko, B, ko, mo, s))
             rc = gate_up(_ptr(lm[4]), _ptr(lm[5]), self.mlp_in[i].data_ptr(), self.h[i].data_ptr(), Fd, H, B, H, Fd, s)
             if rc == _UNSUPPORTED:
-                # refused before any launch: the reference's composition
+                # refused before any launch: the separate projections
                 self.fused_gate_up = False
                 x = self.mlp_in[i].data_ptr()
-                check(gemv(_ptr(lm[4]), x, self._g.data_ptr(), Fd, H, B, H, Fd, s))
-                check(gemv(_ptr(lm[5]), x, self._u.data_ptr(), Fd, H, B, H, Fd, s))
-                torch.mul(F.silu(self._g), self._u, out=self.h[i])
+                w2, y2, m2 = self._gate_up[i]
+                check(group(2, w2, y2, m2, x, H, B, H, s))
+                check(lib.gdsllm_silu_mul(self._g.data_ptr(), self._u.data_ptr(), self.h[i].data_ptr(), B * Fd, s))
             elif rc != 0:
                 check(rc)
             check(gemv(_ptr(lm[6]), self.h[i].data_ptr(), self.down[i].data_ptr(), H, Fd, B, Fd, H, s))
@@ -178,6 +181,5 @@ class DecodeSweep:
 
     @property
     def launches_per_token(self) -> int:
-        """Projection launches per token (the SiLU and product of a refused
-        gate/up/SiLU launch not counted)."""
+        """Launches per token where every group is one launch."""
         return (4 if self.fused_gate_up else 5) * len(self.metas) + 1

@@ -299,6 +299,11 @@ int gdsllm_moe_combine(const void* expert_out, const void* shared_out,
                        const void* shared_gate_logit, void* y,
                        int64_t hidden, int64_t n_tok, void* stream);
 
+/* h[i] = fp16(fp16(silu(gate[i])) * up[i]), i < n, fp16 with torch's rounding:
+ * F.silu(gate) * up of runtime/llama.py:253-256 in one launch.  h may be gate
+ * or up.                                                                     */
+int gdsllm_silu_mul(const void* gate, const void* up, void* h, int64_t n, void* stream);
+
 /* ---------------------------------------------------- prefill dequant-GEMM --
  * Y[t][r] = fp16( sum_k X[t][k] * W[r][k] ), t < tokens, on MFMA.  Replaces
  * the prefill branch dequant -> F.linear (runtime/llama.py:160-166).

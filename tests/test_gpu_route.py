@@ -133,3 +133,30 @@ def test_moe_combine(gpu, H, n):
     if H > 4:
         got = to_np(y)
         assert got[0, 0] == np.float16(65504.0) and np.isnan(got[0, 1]) and got[0, 2] == np.float16(-65504.0)
+
+
+@pytest.mark.parametrize("n,off", [(1, 0), (7, 0), (2048, 0), (2049, 0), (8 * 11008, 0), (3 * 1000003, 0), (4099, 1)])
+def test_silu_mul(gpu, n, off):
+    """fp16(fp16(silu(g)) * u) against the oracle's: one fp16 ulp of silu times
+    |u| plus one ulp of h (the device's expf against numpy's); infinities and
+    NaN as the oracle has them; elements past n stay; h in place of gate gives
+    the same bits."""
+    g, u = (syn.activations(1, n + 16, gen(6900 + n + i)).view(-1) * 4 for i in range(2))
+    if n >= 2048:
+        g[[3, 5, 9]] = torch.tensor([float("inf"), -65504.0, float("nan")], dtype=torch.float16)
+    gd, ud = g.to(gpu), u.to(gpu)
+    h = torch.full((n + 16,), 7.0, dtype=torch.float16, device=gpu)
+    check(capi().gdsllm_silu_mul(ptr(gd[off:]), ptr(ud[off:]), ptr(h[off:]), n, stream()))
+    check(capi().gdsllm_silu_mul(ptr(gd[off:]), ptr(ud[off:]), ptr(gd[off:]), n, stream()))
+    torch.cuda.synchronize()
+    assert torch.equal(gd[off:off + n].view(torch.int16), h[off:off + n].view(torch.int16))
+    hk = to_np(h).astype(np.float64)
+    assert (np.delete(hk, np.s_[off:off + n]) == 7.0).all(), "elements past n were written"
+    gn, un = to_np(g)[off:off + n], to_np(u)[off:off + n]
+    with np.errstate(all="ignore"):
+        sg = oq.silu_fp16(gn)
+        want = (sg.astype(np.float32) * un.astype(np.float32)).astype(np.float16)
+    got, fin = hk[off:off + n], np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    bound = oq.fp16_ulp(sg[fin]) * np.abs(un[fin].astype(np.float64)) + oq.fp16_ulp(want[fin])
+    assert (np.abs(got[fin] - want[fin].astype(np.float64)) <= bound).all()
