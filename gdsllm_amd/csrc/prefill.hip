@@ -806,14 +806,17 @@ __global__ __launch_bounds__(256) void split_sum(const float* __restrict__ part,
 // one more launch and the traffic of the partial sums.  Estimated as in
 // pick_tile, with the constants fitted to launches of one round: 5 us fixed,
 // 22 us x r per 4096 of K, and for a split 4 us plus its partial sums' bytes
-// at 4 TB/s; taken where it saves 5%.  Measured, whole -> split (us): Q8_0
+// at 4 TB/s; taken where it saves 5% and all parts run at once (which also
+// keeps the workspace under 17 MB; 35840 x 6144 gate/up rows at 10 tokens as
+// three rounds of half tiles against two of whole ones: 193 against 192 us for
+// its MLP).  Measured, whole -> split (us): Q8_0
 // 8192 x 28672 at 100 / 256 tokens 190.5 -> 92.5 (128 tokens, 4 parts) / 209
 // -> 177 (128, 2); 8192 x 8192 at 64 / 128 60.8 -> 27.9 (64, 4) / 58.5 -> 37.3
 // (128, 4); 11008 x 4096 at 60 33.5 -> 24.5 (64, 2); Q4_0 4096 x 11008 at 128 /
 // 256 / 333 56.7 -> 27.2 (64, 4) / 57.8 -> 38.7 (128, 4) / 59.1 -> 55.1 (128,
 // 2); 4096 x 4096 at 64 24.9 -> 15.5 (64, 4); 2048 x 4096 at 512 25.4 -> 23.1
 // (64, 2).  4096 x 11008 at 512 (64.6 -> 61.9, 128 tokens, 2 parts) stays whole,
-// and so does every launch whose whole tiles fill the CUs.
+// and so does every launch of over half a round of tiles.
 struct SplitPlan {
     int bt = 0, parts = 1;
 };
@@ -834,7 +837,8 @@ inline SplitPlan pick_split(int64_t M, int64_t T, int64_t K) {
     double cost = whole * 0.95;
     for (int bt : {128, 64})
         for (int s = 2; s <= 8 && units / s >= 4; ++s) {
-            const double c = rounds(jobs(128, bt) * s) * (5.0 + (bt == 128 ? 1.7 : 1.1) * unit / s) + 4.0 +
+            if (jobs(128, bt) * s > cu) break;
+            const double c = 5.0 + (bt == 128 ? 1.7 : 1.1) * unit / s + 4.0 +
                              8.0 * s * static_cast<double>(T) * static_cast<double>(M) / 4e6;
             if (c < cost) {
                 cost = c;
