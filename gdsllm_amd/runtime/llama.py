@@ -27,6 +27,8 @@ from typing import Dict, Optional
 
 import torch
 import torch.nn.functional as F
+from torch._C._functorch import is_functorch_wrapped_tensor
+from torch.autograd import forward_ad
 
 from . import ext
 
@@ -137,13 +139,29 @@ def _gguf_pair(g, u) -> bool:
             g["buffer"].device_id == u["buffer"].device_id)
 
 
+def untransformed(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel that reads and writes raw pointers may stand in for
+    torch ops on these tensors: it is seen by no gradient, forward-mode tangent,
+    torch.func transform, trace or dispatch mode, which would otherwise lose it
+    without an error (a traced function would return uninitialised memory)."""
+    return not (torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or
+                any(type(t) not in (torch.Tensor, torch.nn.Parameter) or t.requires_grad or
+                    is_functorch_wrapped_tensor(t) or forward_ad.unpack_dual(t).tangent is not None for t in tensors))
+
+
 def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """F.silu(gate) * up (runtime/llama.py:253-256): one launch for fp16 on the
-    device, torch's ops otherwise (and where gradients are recorded)."""
+    device, torch's ops otherwise and where they are recorded (untransformed)."""
     if (gate.is_cuda and gate.dtype == up.dtype == torch.float16 and gate.shape == up.shape and
-            gate.device == up.device and not (gate.requires_grad or up.requires_grad)):
+            gate.device == up.device and untransformed(gate, up)):
         return ext().silu_mul(gate, up)
     return F.silu(gate) * up
+
+
+def own_weights(*weights) -> bool:
+    """Weights in this library's formats (GGUF, affine-Q4, per-column int8), not
+    plain tensors, whose whole MLP stays torch's."""
+    return all(isinstance(w, dict) or w.dtype == torch.int8 for w in weights)
 
 
 def mlp(x: torch.Tensor, weights: Dict, scratch: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -167,4 +185,5 @@ def mlp(x: torch.Tensor, weights: Dict, scratch: Optional[torch.Tensor] = None) 
             return dequant_linear(h, weights, "mlp.down_proj", scratch)
     gate = dequant_linear(x, weights, "mlp.gate_proj", scratch)
     up = dequant_linear(x, weights, "mlp.up_proj", scratch)
-    return dequant_linear(silu_mul(gate, up), weights, "mlp.down_proj", scratch)
+    h = silu_mul(gate, up) if own_weights(g, u) else F.silu(gate) * up
+    return dequant_linear(h, weights, "mlp.down_proj", scratch)

@@ -23,7 +23,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ext
-from .llama import FUSED_GEMM_MAX_TOKENS, prefill_takes_fused_gemm, silu_mul
+from .llama import FUSED_GEMM_MAX_TOKENS, own_weights, prefill_takes_fused_gemm, silu_mul, untransformed
 
 
 def _dequant_affine_q4(meta: dict, scratch: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -145,7 +145,7 @@ def _shared_gate_up_silu(x: torch.Tensor, weights: Dict) -> Optional[torch.Tenso
     if not all(isinstance(m, dict) and m.get("quant_type") == "affine_q4" and len(m["shape"]) == 2 for m in (g, u)):
         return None
     if list(g["shape"]) != list(u["shape"]) or g["group_size"] != u["group_size"] or \
-            g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8) or x.requires_grad:
+            g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8) or not untransformed(x):
         return None
     if x.numel() // x.shape[-1] > FUSED_GEMM_MAX_TOKENS and 2 * int(g["shape"][0]) > 8192:
         return None
@@ -250,7 +250,8 @@ def moe_mlp_selective(
     if shared_h is None:
         shared_gate = affine_q4_linear(x, weights, "mlp.shared_expert.gate_proj", scratch)
         shared_up = affine_q4_linear(x, weights, "mlp.shared_expert.up_proj", scratch)
-        shared_h = silu_mul(shared_gate, shared_up)
+        own = own_weights(*(weights[f"{p}.weight"] for p in _SHARED_PROJ[:2]))
+        shared_h = silu_mul(shared_gate, shared_up) if own else F.silu(shared_gate) * shared_up
     shared_out = affine_q4_linear(shared_h, weights, "mlp.shared_expert.down_proj", scratch)
     sg = weights["mlp.shared_expert_gate.weight"]
     if isinstance(sg, dict):
