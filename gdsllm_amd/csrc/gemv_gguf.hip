@@ -1517,11 +1517,11 @@ int launch_q4_codes(const void* w, const uint16_t* x, uint16_t* y, int M, int K,
 // w and w+16 of K, for every 16-row tile the workgroup owns, so its slice of x
 // (up to 2 super-blocks x 8 batch rows, 8 KiB) is loaded once instead of once
 // per tile.  LDS then holds weights only: 4 stage slots per wave (Q8_0: 2, of
-// twice the bytes), so a tile's whole K is in flight at once.  The x slice comes in by LDS DMA (2 batch rows
-// x 512 contiguous bytes per transfer) into the wave's slots and is read into
-// registers before the first weights are issued; register loads straight
-// from HBM gathered 8 batch rows per instruction and took ~4 us longer per
-// launch.
+// twice the bytes), so a tile's whole K is in flight at once.  The x slice
+// comes in by LDS DMA (2 batch rows x 512 contiguous bytes per transfer) into
+// the wave's slots and is read into registers before the weights that take
+// their place are issued; register loads straight from HBM gathered 8 batch
+// rows per instruction and took ~4 us longer per launch.
 namespace bx {
 constexpr int kRT = 16;  // rows per tile
 // WV waves per workgroup, at most NSB super-blocks of K per wave, NS stage
@@ -1559,16 +1559,23 @@ using Tall = Cfg<Fmt::Q4_0, 16, 2, 4>;
 // 20.4; with one tile per CU (4096x4096 at batch 3) 5.45 against 5.17.
 using Half = Cfg<Fmt::Q4_0, 8, 2, 4>;
 // Q8_0: the waves' shares of K go by in_dim alone, so a matrix has the same
-// bits alone and in a group.  in_dim <= 4096: Half's split, 2 slots (78 KiB,
+// bits alone and in a group.  in_dim <= 4096: Half's split, 2 slots (76 KiB,
 // two workgroups per CU); with at most one tile per CU the x slice has LDS of
 // its own (140 KiB), so the tile's weights are in flight while x comes in.
 // in_dim <= 8192: Tall's split with 2 slots.  Both wave counts with twice the
 // slots, 4 waves x 4 slots, and 8 waves x 4 super-blocks were no faster at any
 // of 15 shapes.  Against gguf_gemv_mfma, which takes x in with every stage (as
 // many bytes as its weights) and launches each matrix by itself, batch 3 / 8,
-// us: 11008x4096 15.1 / 15.9 -> 13.7 / 14.3, 32000x4096 35.2 / 38.3 -> 29.8 /
-// 30.4, 28672x8192 58.1 / 66.2 -> 49.8 / 51.4, 14336x5120 22.8 / 25.7 -> 22.4 /
-// 22.9, 1024x8192 8.8 / 10.2 -> 7.5 / 9.5, 8192x8192 19.1 / 20.1 -> 19.6 / 20.0.
+// us: 11008x4096 14.3 / 15.7 -> 13.2 / 14.2, 32000x4096 32.1 / 34.8 -> 28.2 /
+// 29.5, 28672x8192 52.5 / 59.2 -> 46.5 / 47.8, 16384x5120 22.4 / 25.2 -> 21.8 /
+// 22.3, 1024x8192 8.8 / 10.0 -> 7.7 / 9.5, 4096x4096 6.8 / 7.3 -> 6.7 / 7.3.
+// With x always ahead of the first weights, matrices of few tiles or short K
+// lost (256x4352 at batch 8 6.3 -> 7.7, 5120x2048 7.4 -> 8.1), hence the two
+// orders below: 6.1 and 6.9.  What is left is two or three even rounds of tiles
+// over in_dim past 4096 at batch 3-5, 2-5% slower than that kernel by
+// themselves (8192x8192 17.7 -> 18.7 / 19.8 -> 19.4, 8192x4352 11.4 -> 12.0 /
+// 12.6 -> 12.3), and taken because a group has to have the same bits: q/k/v of
+// 8192x8192 51.3 -> 42.0 / 58.2 -> 43.2, of 4096x4096 20.3 -> 14.3 / 21.6 -> 14.8.
 // Past 8192 a wave's x slice is longer than its weights' gain: 4096x11008 14.3
 // / 16.8 against 15.7 / 19.4 with 8 waves x 8 super-blocks, so those keep it.
 using Q8Half = Cfg<Fmt::Q8_0, 8, 2, 2>;
@@ -1622,9 +1629,8 @@ __device__ __forceinline__ Tile tile_of(const Target& tg, int t) {
 }  // namespace bx
 
 template <class C, int MODE>
-__global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_xreg(const bx::Target tg,
-                                                                    const uint16_t* __restrict__ X, int K, int nb,
-                                                                    int64_t ldx) {
+__global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_xreg(const bx::Target tg, const uint16_t* __restrict__ X,
+                                                                 int K, int nb, int64_t ldx) {
     constexpr Fmt F = C::kFmt;
     static_assert(F == Fmt::Q4_0 || MODE != 2, "gate/up pairs are Q4_0");
     constexpr int RT = bx::kRT, NRG = RT / 8, NS = C::kNS, kCh = C::kCh, kSb = C::kSb;
@@ -1756,51 +1762,81 @@ __global__ __launch_bounds__(C::kWaves * 64) void gguf_gemv_xreg(const bx::Targe
         return;
     }
 
-    // x slice: 4 transfers per super-block into the wave's slots (transfer jj
-    // holds batch rows 2jj, 2jj+1, rows past nb repeat row nb - 1; 2 where
-    // nb <= 4; the super-blocks past this wave's last repeat it), then into
-    // registers.
+    // x slice: 4 transfers per super-block of this wave (transfer jj holds batch
+    // rows 2jj, 2jj+1, rows past nb repeat row nb - 1; 2 where nb <= 4) into
+    // LDS, then into registers.
     half8_t xa[C::kNSB][4];
     int issued = min(Q, NS);  // stages of weights issued
-    {
-        const int nxt = nb <= 4 ? 2 : 4;
-        const uint32_t xs = C::kXSep ? lds0 + C::kXOff + wave * C::kXBytes : slot0;
+    const int nxt = nb <= 4 ? 2 : 4;
+    auto load_x = [&](int s2, uint32_t at) {
+        const int sb = wave + C::kWaves * s2;
 #pragma unroll
-        for (int s2 = 0; s2 < C::kNSB; ++s2) {
-            const int sb = wave + C::kWaves * min(s2, nst - 1);
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                if (jj >= nxt) break;
-                const int tr = min(2 * jj + (lane >> 5), nb - 1);
-                dma16_asm(static_cast<uint32_t>(2 * (tr * ldx + 8 * (lane & 31))), X + 256 * sb,
-                          xs + 4096 * s2 + 1024 * jj);
-            }
+        for (int jj = 0; jj < 4; ++jj) {
+            if (jj >= nxt) break;
+            const int tr = min(2 * jj + (lane >> 5), nb - 1);
+            dma16_asm(static_cast<uint32_t>(2 * (tr * ldx + 8 * (lane & 31))), X + 256 * sb, at + 1024 * jj);
         }
-        if constexpr (C::kXSep) {
-            // x went out first: wait for all but the weights' transfers
-            static_assert(NS == 2, "one or two stages issued");
-            for (int q = 0; q < issued; ++q) issue();
-            if (issued == 2) wait_vmcnt_asm<2 * NWD>();
-            else wait_vmcnt_asm<NWD>();
-        } else {
-            wait_vmcnt_asm<0>();
-        }
+    };
+    auto read_x = [&](int s2, uint32_t at) {
         // lane (g, j): batch row j & 7 of block 2p + par, elements 4g.. and 16+4g..
         const int t = min(j & 7, nb - 1);
-        const uint8_t* xl = lds + (xs - lds0) + (t >> 1) * 1024 + (t & 1) * 512 + 2 * (32 * par + 4 * g);
+        const uint8_t* xl = lds + (at - lds0) + (t >> 1) * 1024 + (t & 1) * 512 + 2 * (32 * par + 4 * g);
 #pragma unroll
-        for (int s2 = 0; s2 < C::kNSB; ++s2)
+        for (int p = 0; p < 4; ++p) {
+            const uint2 lo = *reinterpret_cast<const uint2*>(xl + 128 * p);
+            const uint2 hi = *reinterpret_cast<const uint2*>(xl + 128 * p + 32);
+            xa[s2][p] = __builtin_bit_cast(half8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
+        }
+    };
+    // the reads have returned before transfers overwrite the slots
+    auto x_read = [&]() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+    // into the wave's slots, before its first weights
+    auto x_then_w = [&]() {
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                const uint2 lo = *reinterpret_cast<const uint2*>(xl + 4096 * s2 + 128 * p);
-                const uint2 hi = *reinterpret_cast<const uint2*>(xl + 4096 * s2 + 128 * p + 32);
-                xa[s2][p] = __builtin_bit_cast(half8_t, make_uint4(lo.x, lo.y, hi.x, hi.y));
-            }
-        // the reads have returned before transfers overwrite the slots
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-    if constexpr (!C::kXSep)
+        for (int s2 = 0; s2 < C::kNSB; ++s2) load_x(min(s2, nst - 1), slot0 + 4096 * s2);
+        wait_vmcnt_asm<0>();
+#pragma unroll
+        for (int s2 = 0; s2 < C::kNSB; ++s2) read_x(s2, slot0 + 4096 * s2);
+        x_read();
         for (int q = 0; q < issued; ++q) issue();
+    };
+    if constexpr (F == Fmt::Q4_0) {
+        x_then_w();
+    } else {
+        // x into LDS of its own, or the second slot until it is in registers,
+        // with the first weights in flight beside it, where most waves have
+        // one super-block.  (Two: the second stage's weights would wait for x,
+        // and at batch 5-8 the slot holds one super-block of x at a time,
+        // which is worth it only for the few of 16 waves that have two.)
+        static_assert(C::kNSB == 2 && NS == 2, "one or two super-blocks and stages");
+        const uint32_t xs = C::kXSep ? lds0 + C::kXOff + wave * C::kXBytes : slot0 + C::kSlotBytes;
+        const uint32_t xs1 = xs + 1024 * nxt;
+        const bool both = C::kXSep || nst == 1 || nxt == 2;  // all of the slice at once
+        const bool few = 2 * S <= 3 * C::kWaves && (both || C::kWaves == 16);  // of the waves have two
+        if (!C::kXSep && nst == 2 && !few) {
+            x_then_w();
+        } else {
+            load_x(0, xs);
+            if (both && nst == 2) load_x(1, xs1);
+            issue();
+            if (C::kXSep && issued == 2) {
+                issue();
+                wait_vmcnt_asm<2 * NWD>();
+            } else {
+                wait_vmcnt_asm<NWD>();
+            }
+            read_x(0, xs);
+            if (both && nst == 2) read_x(1, xs1);
+            x_read();
+            if (!both) {
+                load_x(1, xs);
+                wait_vmcnt_asm<0>();
+                read_x(1, xs);
+                x_read();
+            }
+            if (!C::kXSep && issued == 2) issue();
+        }
+    }
 
     const half8_t kneg = {static_cast<half_t>(-1032.0f), static_cast<half_t>(-1032.0f), static_cast<half_t>(-1032.0f),
                           static_cast<half_t>(-1032.0f), static_cast<half_t>(-72.0f),   static_cast<half_t>(-72.0f),

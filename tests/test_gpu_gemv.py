@@ -232,6 +232,37 @@ def test_gemv_group(gpu, fmt, Ms, K, B):
         assert not bad.any(), f"group[{i}]: {int(bad.sum())} outputs apart beyond reassociation"
 
 
+# (M, K, B) of the Q8_0 x-in-registers kernel by how x comes in: LDS of its own
+# (at most one 16-row tile per compute unit, in_dim <= 4096); the second slot,
+# with the first weights in flight (8 waves of up to 8 and up to 12 super-blocks,
+# 16 waves of 17-24, one or two of them per wave, both or one at a time); both
+# slots, ahead of the weights (8 waves of 9-12 and 13-16, 16 waves of 25-32).
+Q8_XREG_CASES = [(33, 256, 8), (33, 2304, 5), (33, 4096, 8), (4100, 256, 5), (4100, 2048, 8), (4100, 3072, 4),
+                 (4100, 2560, 6), (4100, 4096, 3), (4100, 3840, 8), (37, 4352, 8), (37, 4352, 3), (37, 5120, 5),
+                 (4100, 4608, 4), (37, 6144, 8), (37, 6400, 3), (37, 6400, 8), (37, 7936, 6), (4100, 8192, 4)]
+
+
+@pytest.mark.parametrize("M,K,B", Q8_XREG_CASES, ids=[f"{m}x{k}_b{b}" for m, k, b in Q8_XREG_CASES])
+def test_q8_xreg_x_orders(gpu, M, K, B):
+    """Within the GEMV tolerance of the oracle, the same bits as in a group of
+    two (whose tiles may take x in by another order), nothing written past the
+    rows."""
+    import ctypes
+
+    w, x, deq = _gguf_case("q8_0", M, K, B, 6700 + M + K + B)
+    wd, xd = w.to(gpu), x.to(gpu)
+    y = torch.full((B, M + 3), 7.0, dtype=torch.float16, device=gpu)
+    check(capi().gdsllm_fused_q8_0_gemv(ptr(wd), ptr(xd), ptr(y), M, K, B, K, M + 3, stream()))
+    ys = [torch.empty(B, M, dtype=torch.float16, device=gpu) for _ in range(2)]
+    check(capi().gdsllm_fused_q8_0_gemv_group(2, (ctypes.c_void_p * 2)(ptr(wd), ptr(wd)),
+                                              (ctypes.c_void_p * 2)(*[ptr(t) for t in ys]),
+                                              (ctypes.c_int64 * 2)(M, M), ptr(xd), K, B, K, stream()))
+    torch.cuda.synchronize()
+    assert bool((y[:, M:] == 7.0).all()), "columns past the rows were written"
+    assert_gemv_close(to_np(y[:, :M].contiguous()), deq, to_np(x), f"q8_0 {M}x{K} B{B}")
+    assert all(torch.equal(t, y[:, :M]) for t in ys), "a group's bits differ from the single GEMV's"
+
+
 # Fewer row groups than compute units and in_dim over 2-4 windows of 4096:
 # the single-matrix launch splits the windows over waves (2 windows; 3 with a
 # ragged last one; 4), and a group of two matrices keeps them in one wave.
