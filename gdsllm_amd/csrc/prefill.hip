@@ -64,6 +64,8 @@
 //             gate and up outputs never reach HBM.
 
 #include <algorithm>
+#include <climits>
+#include <cmath>
 
 #include "moe_stream.h"
 
@@ -937,17 +939,28 @@ int dense_dual_gemm_auto(const GemmArgs& a, void* workspace, size_t bytes, hipSt
 // moe_sort (one workgroup): the T*k routed (token, slot) entries sorted by
 // expert.  tok[p] is the token of position p, pos[t*k + j] the position of
 // entry (t, j) (-1 for an expert index outside [0, E)), tiles[] the
-// (expert, p0, n) token tiles of at most BT positions, *ntiles their count.
-// The order of positions inside one expert is not fixed (LDS atomics); each
-// output row depends only on its own token and expert, so results are.
+// (expert, p0, n) token tiles of at most BT positions.  The order of positions
+// inside one expert is not fixed (LDS atomics); each output row depends only
+// on its own token and expert, so results are.
+// counts[0] is the number of tiles.  Whether the chunk runs on the split-K
+// tiles or as weight streams (moe_stream.hip) is settled here, where the load of
+// every expert is known: counts[1] is the number of tiles for the former, 0
+// where the latter take the chunk; counts[2] is the number of passes of at
+// most kStreamTokens positions for the streams, or 0, with the tiles of two
+// passes first in the list, counts[3] of them.
+struct MoePath {
+    int min_passes;  // fewest passes that run as streams (INT_MAX: the tiles)
+    int num, den;    // and at most num / den of them per tile
+};
 constexpr int kSortThreads = 1024;
 constexpr int kSortMaxExperts = 4096;
 
 __global__ __launch_bounds__(kSortThreads) void moe_sort(const int32_t* __restrict__ idx, int n_entries, int top_k,
-                                                         int E, int BT, int* __restrict__ tok, int* __restrict__ pos,
-                                                         int4* __restrict__ tiles, int* __restrict__ ntiles) {
-    __shared__ int cnt[kSortMaxExperts], off[kSortMaxExperts], toff[kSortMaxExperts];
-    __shared__ int part[kSortThreads], tpart[kSortThreads];
+                                                         int E, int BT, MoePath path, int* __restrict__ tok,
+                                                         int* __restrict__ pos, int4* __restrict__ tiles,
+                                                         int* __restrict__ counts) {
+    __shared__ int cnt[kSortMaxExperts], off[kSortMaxExperts];
+    __shared__ int wsum[3][kSortThreads / 64];  // the waves' sums
     const int tid = threadIdx.x;
     for (int e = tid; e < E; e += kSortThreads) cnt[e] = 0;
     __syncthreads();
@@ -956,37 +969,60 @@ __global__ __launch_bounds__(kSortThreads) void moe_sort(const int32_t* __restri
         if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
     }
     __syncthreads();
-    // exclusive scans of the counts and of the tile counts: each thread sums a
-    // contiguous run of experts, then a scan over the threads
+    // exclusive scans of the counts, of the tile counts and of the counts of
+    // two-pass tiles: each thread sums a contiguous run of experts
     const int per = (E + kSortThreads - 1) / kSortThreads;
     const int e0 = min(E, tid * per), e1 = min(E, e0 + per);
-    int sc = 0, st = 0;
+    auto two_pass = [&](int c) { return c / BT + (c % BT > kStreamTokens ? 1 : 0); };
+    int sc = 0, st = 0, sb = 0;
     for (int e = e0; e < e1; ++e) {
         sc += cnt[e];
         st += (cnt[e] + BT - 1) / BT;
+        sb += two_pass(cnt[e]);
     }
-    part[tid] = sc;
-    tpart[tid] = st;
+    // inclusive scans over the wave's threads, then over the 16 waves' sums
+    const int lane = tid & 63, wave = tid >> 6;
+    int ic = sc, it = st, ib = sb;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int vc = __shfl_up(ic, d, 64), vt = __shfl_up(it, d, 64), vb = __shfl_up(ib, d, 64);
+        if (lane >= d) ic += vc, it += vt, ib += vb;
+    }
+    if (lane == 63) wsum[0][wave] = ic, wsum[1][wave] = it, wsum[2][wave] = ib;
     __syncthreads();
-    for (int d = 1; d < kSortThreads; d <<= 1) {
-        const int pc = tid >= d ? part[tid - d] : 0, pt = tid >= d ? tpart[tid - d] : 0;
-        __syncthreads();
-        part[tid] += pc;
-        tpart[tid] += pt;
-        __syncthreads();
+    int ntiles = 0, ntwo = 0;
+#pragma unroll
+    for (int w = 0; w < kSortThreads / 64; ++w) {
+        if (w == wave) it += ntiles, ib += ntwo;
+        if (w < wave) ic += wsum[0][w];
+        ntiles += wsum[1][w];
+        ntwo += wsum[2][w];
     }
-    int rc = part[tid] - sc, rt = tpart[tid] - st;
+    const int passes = ntiles + ntwo;
+    const bool streams = passes >= path.min_passes &&
+                         static_cast<int64_t>(passes) * path.den <= static_cast<int64_t>(ntiles) * path.num;
+    if (tid == 0) {
+        counts[0] = ntiles;
+        counts[1] = streams ? 0 : ntiles;
+        counts[2] = streams ? passes : 0;
+        counts[3] = ntwo;
+    }
+    // this thread's experts: first position, first tile and first two-pass tile
+    int rc = ic - sc, rt = it - st, rb = ib - sb;
     for (int e = e0; e < e1; ++e) {
+        const int c = cnt[e];
         off[e] = rc;
-        toff[e] = rt;
-        rc += cnt[e];
-        rt += (cnt[e] + BT - 1) / BT;
-    }
-    if (tid == kSortThreads - 1) *ntiles = tpart[tid];
-    __syncthreads();
-    for (int e = tid; e < E; e += kSortThreads) {
-        const int c = cnt[e], o = off[e];
-        for (int j = 0; j * BT < c; ++j) tiles[toff[e] + j] = int4{e, o + j * BT, min(BT, c - j * BT), 0};
+        for (int p = 0; p < c; p += BT) {
+            const int n = min(BT, c - p);
+            int at = rt++;
+            if (streams) {
+                const bool two = n > kStreamTokens;
+                at = two ? rb : ntwo + at - rb;  // rb two-pass tiles come before this one
+                rb += two ? 1 : 0;
+            }
+            tiles[at] = int4{e, rc + p, n, 0};
+        }
+        rc += c;
         cnt[e] = 0;  // reused as the fill cursor
     }
     __syncthreads();
@@ -1038,17 +1074,40 @@ __global__ __launch_bounds__(256) void moe_prefill_combine(const uint16_t* __res
 }
 
 constexpr int kMoeBT = 32;
-// Mean tokens per expert up to which the chunk runs as weight streams
-// (moe_stream.hip) instead of the split-K tiles below: a stream pass serves 16
-// tokens of an expert, the tiles 32 for one dequantization.  Measured, us per
-// chunk with the shared expert, tiles against streams: 512 experts of 1024 x
-// 4096 at a mean of 1 / 5 / 10 / 14 / 18 tokens 701 / 1055 / 1107 / 1154 / 1187
-// against 510 / 729 / 815 / 1012 / 1278; 256 of 768 x 3072 at 5 / 10 / 14 / 18
-// 349 / 372 / 387 / 400 against 254 / 342 / 379 / 449; 128 of 512 x 2048 at 5 /
-// 10 / 14 / 18 137 / 143 / 141 / 150 against 108 / 142 / 141 / 162; 64 of 1024
-// x 4096, whose few jobs leave the longest expert as the tail, at 5 / 10 / 14
-// 197 / 199 / 203 against 145 / 205 / 207.
-inline int64_t stream_tokens(int64_t experts) { return experts >= 128 ? 10 : 8; }
+// What moe_sort settles the path of a chunk by.  Streams pay while an expert's
+// entries take few passes of 16 more than tiles of 32, and where the two
+// launches have jobs for every compute unit: below that one job's length is the
+// time of the launch, and the tiles have four times as many.  Measured with
+// weights out of the caches, us per chunk, tiles / streams (n: passes):
+//   1024 x 4096  n 8: 46 / 79   26: 74 / 79   33: 94 / 78   66: 162 / 151
+//                118: 251 / 168   511: 1019 / 700
+//   768 x 3072   n 25: 53 / 65   45: 81 / 68   91: 122 / 117   246: 301 / 198
+//   512 x 2048   n 8: 31 / 52   48: 47 / 50   70: 61 / 54   128: 92 / 65
+//   1280 x 2048  n 8: 31 / 60   32: 60 / 67   40: 69 / 66   54: 86 / 86
+// and over 1024 x 4096 at 1.1 / 1.25 / 1.5 / 2 passes per tile 865 / 634, 1078 /
+// 895, 1125 / 1064 and 518 / 608.  Where the host knows the answer (even routing
+// at random would leave too few passes, or the mean load is past 16) only the
+// tiles are launched; else the pair of launches that moe_sort leaves empty
+// takes 3 us, up to 11 where the empty tile grid is large.
+inline MoePath moe_path(int64_t T, int64_t k, int64_t E, int64_t H, int64_t Fd) {
+    const MoePath tiles{INT_MAX, 0, 1};
+    if (!moe_stream_fits(Fd, H) || !moe_stream_fits(H, Fd) || T * k > kStreamTokens * E) return tiles;
+    const int jobs = moe_stream_jobs(Fd, true) + moe_stream_jobs(H, false);
+    const int min_passes = (cu_count() + jobs - 1) / jobs;
+    const double e = static_cast<double>(E), miss = 1.0 - std::min(1.0, static_cast<double>(k) / e);
+    if (e * (1.0 - std::pow(miss, static_cast<double>(T))) < min_passes) return tiles;
+    return {min_passes, 27, 20};
+}
+
+// Most tiles the split-K launches can get: of n entries over E experts, and
+// where streams are the other choice, fewer than min_passes or a share ntwo /
+// tiles > (num - den) / den of two-pass tiles, of 17 entries or more each.
+inline int64_t max_gemm_tiles(const MoePath& path, int64_t n, int64_t E) {
+    const int64_t all = n / kMoeBT + std::min<int64_t>(E, n);
+    if (path.min_passes == INT_MAX) return all;
+    const int64_t loaded = n * path.den / (path.den + kStreamTokens * (path.num - path.den));
+    return std::min(all, std::max<int64_t>(path.min_passes, loaded));
+}
 
 struct PrefillLayout {
     size_t tok, pos, tiles, ntiles, h, d, total;
@@ -1084,13 +1143,14 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     int* tok = reinterpret_cast<int*>(ws + L.tok);
     int* pos = reinterpret_cast<int*>(ws + L.pos);
     int4* tiles = reinterpret_cast<int4*>(ws + L.tiles);
-    int* ntiles = reinterpret_cast<int*>(ws + L.ntiles);
+    int* counts = reinterpret_cast<int*>(ws + L.ntiles);
+    const MoePath path = moe_path(T, k, E, H, Fd);
     uint16_t* hbuf = reinterpret_cast<uint16_t*>(ws + L.h);
     uint16_t* dbuf = reinterpret_cast<uint16_t*>(ws + L.d);
     hipLaunchKernelGGL(moe_sort, dim3(1), dim3(kSortThreads), 0, stream, idx, static_cast<int>(n), static_cast<int>(k),
-                       static_cast<int>(E), kMoeBT, tok, pos, tiles, ntiles);
+                       static_cast<int>(E), kMoeBT, path, tok, pos, tiles, counts);
     if (int rc = check_hip(hipGetLastError(), "moe_sort launch")) return rc;
-    const int64_t max_tiles = n / kMoeBT + std::min<int64_t>(E, n);
+    const int64_t max_tiles = max_gemm_tiles(path, n, E);
     auto combine = [&]() {
         const int64_t threads = T * (H / 8);
         hipLaunchKernelGGL(moe_prefill_combine, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
@@ -1098,7 +1158,8 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
                            static_cast<int>(T), static_cast<uint16_t*>(y), ldy);
         return check_hip(hipGetLastError(), "moe_prefill_combine launch");
     };
-    if (n <= stream_tokens(E) * E && moe_stream_fits(Fd, H) && moe_stream_fits(H, Fd)) {
+    if (path.min_passes != INT_MAX) {
+        const int64_t max_passes = n / kStreamTokens + std::min<int64_t>(E, n);
         auto pool = [](const gdsllm_affine_experts& p, const gdsllm_affine_experts& p2) {
             MoeStreamArgs a{};
             a.w = static_cast<const uint8_t*>(p.weight);
@@ -1121,17 +1182,16 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
         a.y = hbuf;
         a.ldy = Fd;
         a.tiles = tiles;
-        a.ntiles = ntiles;
-        if (int rc = moe_stream(a, static_cast<int>(g.group_size), true, max_tiles, stream)) return rc;
+        a.passes = counts + 2;
+        if (int rc = moe_stream(a, static_cast<int>(g.group_size), true, max_passes, stream)) return rc;
         MoeStreamArgs b = pool(d, d);
         b.x = hbuf;  // h rows by position
         b.ldx = Fd;
         b.y = dbuf;
         b.ldy = H;
         b.tiles = tiles;
-        b.ntiles = ntiles;
-        if (int rc = moe_stream(b, static_cast<int>(g.group_size), false, max_tiles, stream)) return rc;
-        return combine();
+        b.passes = counts + 2;
+        if (int rc = moe_stream(b, static_cast<int>(g.group_size), false, max_passes, stream)) return rc;
     }
 
     GemmArgs a{};
@@ -1153,7 +1213,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     a.ldy = Fd;
     a.mtiles = static_cast<int>((Fd + 63) / 64);
     a.tiles = tiles;
-    a.ntiles = ntiles;
+    a.ntiles = counts + 1;
     a.tok = tok;
     if (int rc = launch_sk<F, kMoeBT, kDualSilu>(a, static_cast<unsigned>(max_tiles * a.mtiles), stream)) return rc;
 
@@ -1176,7 +1236,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     b.ldy = H;
     b.mtiles = static_cast<int>((H + kBM - 1) / kBM);
     b.tiles = tiles;
-    b.ntiles = ntiles;
+    b.ntiles = counts + 1;
     b.tok = nullptr;
     if (int rc = launch_sk<F, kMoeBT, kGather>(b, static_cast<unsigned>(max_tiles * b.mtiles), stream)) return rc;
     return combine();

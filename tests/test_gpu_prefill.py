@@ -7,13 +7,15 @@ The dense GEMMs replace the reference's prefill route dequant -> F.linear
 replaces the per-expert loop of runtime/qwen_moe.py:475-492.
 """
 
+import ctypes
+import itertools
 
 import numpy as np
 import pytest
 import torch
 
-from helpers import (affine_dequant_np, assert_gemv_close, capi, check, check_moe_prefill, check_sort, gen, moe_prefill,
-                     oq, ptr, stream, syn, to_np)
+from helpers import (affine_dequant_np, assert_gemv_close, capi, check, check_moe_prefill, check_sort, experts_struct,
+                     gen, moe_prefill, oq, prefill_layout, ptr, stream, syn, to_np)
 
 pytestmark = pytest.mark.gpu
 
@@ -264,6 +266,76 @@ def test_moe_prefill_few_tokens_per_expert(gpu, E, H, F, g, k, T):
     check_sort(idx, tok, pos, tiles, E)
     check_moe_prefill(y, tok, pos, hbuf, dbuf, *pools, x, idx, to_np(wts), g, E,
                       sample=sorted(set(range(0, T, 7)) | {15 % T, 16 % T, T - 1}))
+
+
+def _moe_paths(dev, xd, idx_d, wts_d, g, T, k):
+    """The chunk's outputs and (tiles, tiles of the split-K launches, passes of
+    the stream launches, two-pass tiles) as the device settled them."""
+    gs, us, ds = (experts_struct(*p, g) for p in dev)
+    E, F, H = gs.num_experts, gs.out_dim, gs.in_dim
+    L = prefill_layout(T, k, F, H, E)
+    ws = torch.zeros(L["total"], dtype=torch.uint8, device=xd.device)
+    y = torch.full((T, H), 3.0, dtype=torch.float16, device=xd.device)
+    check(capi().gdsllm_moe_prefill_affine_q4(ctypes.byref(gs), ctypes.byref(us), ctypes.byref(ds), ptr(xd), H,
+                                              ptr(idx_d), ptr(wts_d), T, k, ptr(y), H, ptr(ws), L["total"], stream()))
+    torch.cuda.synchronize()
+    return y, to_np(ws[L["ntiles"]:L["ntiles"] + 16].view(torch.int32)).tolist()
+
+
+# (E, H, F, g, k, T, loads, streams): the first slots of the tokens go round
+# robin over experts 0 .. len(loads)-1 until expert i has loads[i] of them; the
+# other slots go over the rest in turn.  Streams with tiles of one and two
+# passes (17, 31, 32, 33 and 48 tokens), one or two jobs per pass, rows past a
+# job's range (H = 1280), K of 256 .. 2048 and every group size; then the same
+# pools with the load on a few experts or too few passes, which the device gives
+# to the split-K tiles; then what the host gives to them by itself: a mean load
+# past 16, few experts, a hidden size no stream takes.
+PATH_CASES = [
+    (60, 2048, 1024, 64, 3, 60, (17, 31), True), (180, 256, 256, 32, 4, 80, (32, 33), True),
+    (80, 1536, 512, 128, 3, 70, (48,), True), (70, 1280, 768, 64, 2, 100, (16, 1), True),
+    (150, 768, 256, 64, 3, 120, (), True), (110, 1024, 512, 32, 3, 90, (40,), True),
+    (60, 2048, 1024, 64, 3, 60, None, False), (180, 256, 256, 32, 4, 80, None, False),
+    (60, 2048, 1024, 32, 3, 39, "few", False),
+    (6, 1024, 256, 32, 3, 40, (), False), (4, 4096, 1024, 64, 2, 70, (33,), False), (60, 4608, 256, 32, 2, 70, (), False),
+]
+
+
+@pytest.mark.parametrize("bad", [False, True], ids=["", "out_of_range"])
+@pytest.mark.parametrize("E,H,F,g,k,T,loads,streams", PATH_CASES,
+                         ids=[f"E{c[0]}_H{c[1]}_F{c[2]}_g{c[3]}_T{c[5]}_{'streams' if c[7] else 'tiles'}{i}"
+                              for i, c in enumerate(PATH_CASES)])
+def test_moe_prefill_paths(gpu, E, H, F, g, k, T, loads, streams, bad):
+    """Both forms of the grouped MoE products against the oracle, and which one
+    the chunk's routing gives it: the streams where their passes are enough and
+    at most 1.35 per tile, the split-K tiles else.  With an out-of-range entry
+    in the first token's last slot."""
+    gg = gen(7900 + E + T)
+    pools = [syn.affine_q4_weights(s, g, gg) for s in ([E, F, H], [E, F, H], [E, H, F])]
+    x = syn.activations(T, H, gen(7901 + T))
+    idx = np.empty((T, k), np.int32)
+    if loads is None:       # every token picks the same experts
+        idx[:] = np.arange(3, 3 + k)
+    elif loads == "few":    # three experts short of the fewest passes
+        idx[:] = np.arange(T * k).reshape(T, k) % 39
+    else:
+        first = [e for e, n in enumerate(loads) for _ in range(n)]
+        rest = itertools.cycle(range(len(loads), E))
+        for t in range(T):
+            idx[t] = [first[t] if j == 0 and t < len(first) else next(rest) for j in range(k)]
+    if bad:
+        idx[0, -1] = E + 5
+    wts = torch.softmax(torch.randn(T, k, generator=gen(7902)), -1).to(torch.float16)
+    dev = [tuple(t.to(gpu) for t in p) for p in pools]
+    xd, idx_d, wts_d = x.to(gpu), torch.from_numpy(idx).to(gpu), wts.to(gpu)
+    counts = np.bincount(idx[(idx >= 0) & (idx < E)], minlength=E)
+    ntiles, passes = (int((-(-counts // n)).sum()) for n in (32, 16))
+    y2, path = _moe_paths(dev, xd, idx_d, wts_d, g, T, k)
+    assert path == ([ntiles, 0, passes, passes - ntiles] if streams else [ntiles, ntiles, 0, passes - ntiles])
+    y, tok, pos, tiles, hbuf, dbuf = moe_prefill(*dev, xd, idx_d, wts_d, g, T, k)
+    check_sort(idx, tok, pos, tiles, E)
+    check_moe_prefill(y, tok, pos, hbuf, dbuf, *pools, x, idx, to_np(wts), g, E,
+                      sample=sorted(set(range(0, T, 9)) | {0, 15 % T, 16 % T, T - 1}))
+    assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
 def test_moe_prefill_out_of_range_experts(gpu):
