@@ -358,10 +358,15 @@ extern "C" int gdsllm_silu_mul(const void* gate, const void* up, void* h, int64_
     if (!gate || !up || !h) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, nm + ": null pointer");
     const uintptr_t bits = reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up) | reinterpret_cast<uintptr_t>(h);
     if (bits % 2) return set_error(GDSLLM_ERR_INVALID_ARGUMENT, nm + ": pointers must be 2-byte aligned");
-    const dim3 grid(static_cast<unsigned>((n + 2047) / 2048));
     const auto *g = static_cast<const uint16_t*>(gate), *u = static_cast<const uint16_t*>(up);
-    if (bits % 16 == 0) hipLaunchKernelGGL(silu_mul<true>, grid, dim3(256), 0, as_stream(stream), g, u, static_cast<uint16_t*>(h), n);
-    else hipLaunchKernelGGL(silu_mul<false>, grid, dim3(256), 0, as_stream(stream), g, u, static_cast<uint16_t*>(h), n);
-    if (int rc = check_hip(hipGetLastError(), "silu_mul launch")) return rc;
+    auto* hp = static_cast<uint16_t*>(h);
+    const int64_t most = int64_t(1) << 34;  // elements of one launch: 2^31 threads, of fewer than 2^32
+    for (int64_t i = 0; i < n; i += most) {
+        const int64_t c = std::min(most, n - i);
+        const dim3 grid(static_cast<unsigned>((c + 2047) / 2048));
+        if (bits % 16 == 0) hipLaunchKernelGGL(silu_mul<true>, grid, dim3(256), 0, as_stream(stream), g + i, u + i, hp + i, c);
+        else hipLaunchKernelGGL(silu_mul<false>, grid, dim3(256), 0, as_stream(stream), g + i, u + i, hp + i, c);
+        if (int rc = check_hip(hipGetLastError(), "silu_mul launch")) return rc;
+    }
     return ok();
 }

@@ -160,3 +160,23 @@ def test_silu_mul(gpu, n, off):
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     bound = oq.fp16_ulp(sg[fin]) * np.abs(un[fin].astype(np.float64)) + oq.fp16_ulp(want[fin])
     assert (np.abs(got[fin] - want[fin].astype(np.float64)) <= bound).all()
+
+
+def test_silu_mul_past_one_launch(gpu):
+    """More elements than one launch's threads cover (2^35 + 9, 64 GiB): the
+    ones on both sides of each launch's end and of the call's."""
+    n = 2 ** 35 + 9
+    if torch.cuda.mem_get_info(gpu)[0] < 2 * n + (8 << 30):
+        pytest.skip("needs 72 GiB of free device memory")
+    x = torch.zeros(n + 16, dtype=torch.float16, device=gpu)
+    at = [0, 2 ** 34 - 1, 2 ** 34, 2 ** 35 - 1, 2 ** 35, n - 1, n, n + 15]
+    v = [1.0, -2.0, 3.0, 0.5, -0.25, 4.0, 5.0, 6.0]
+    for i, e in zip(at, v):
+        x[i] = e
+    check(capi().gdsllm_silu_mul(ptr(x), ptr(x), ptr(x), n, stream()))
+    torch.cuda.synchronize()
+    got = torch.stack([x[i] for i in at]).double().cpu()
+    assert got[6:].tolist() == v[6:], "elements past n were written"
+    want = torch.tensor(v[:6], dtype=torch.float64)
+    want = torch.nn.functional.silu(want) * want
+    assert bool(((got[:6] - want).abs() <= want.abs() * 2.0 ** -9).all())  # one ulp of silu and one of the product
