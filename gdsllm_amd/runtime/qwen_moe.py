@@ -134,20 +134,28 @@ def _entry(m: dict) -> tuple:
     return (m["buffer"], list(m["shape"]), m["weight_offset"], m["scale_offset"], m["bias_offset"], m["group_size"])
 
 
+_SHARED_FUSED_MAX = 1 << 23  # gate and up outputs of a chunk past 512 tokens
+
+
 def _shared_gate_up_silu(x: torch.Tensor, weights: Dict) -> Optional[torch.Tensor]:
     """h = silu(gate x) * (up x) of the shared expert of a prefill chunk
     (runtime/qwen_moe.py:497-505) in one MFMA launch, split along K where its
-    tiles are few (512 tokens over 1024 x 4096: 29 us, against 60 us as two
-    dequants, two GEMMs and the elementwise ops).  Long chunks over many rows
-    keep the separate route, which dequantizes once per call (the line of
-    prefill_takes_fused_gemm).  None where the launch does not apply."""
+    tiles are few, against two dequants, two GEMMs and the elementwise op.
+    Long chunks over many rows keep the separate route, which dequantizes once
+    per call.  None where the launch does not apply.
+
+    Separate / fused, us: 1024 x 4096 at 9 / 128 / 512 / 2048 / 4096 tokens 37 /
+    18, 46 / 21, 53 / 27, 74 / 46, 99 / 86; 256 x 2048 at 9 / 512 32 / 18, 33 /
+    19; 2048 x 4096 at 2048 / 4096 98 / 86, 162 / 168; 4096 x 4096 at 1024 /
+    2048 101 / 88, 164 / 171."""
     g, u = (weights.get(f"{p}.weight") for p in _SHARED_PROJ[:2])
     if not all(isinstance(m, dict) and m.get("quant_type") == "affine_q4" and len(m["shape"]) == 2 for m in (g, u)):
         return None
     if list(g["shape"]) != list(u["shape"]) or g["group_size"] != u["group_size"] or \
             g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8) or not untransformed(x):
         return None
-    if x.numel() // x.shape[-1] > FUSED_GEMM_MAX_TOKENS and 2 * int(g["shape"][0]) > 8192:
+    tokens, rows = x.numel() // x.shape[-1], 2 * int(g["shape"][0])
+    if tokens > FUSED_GEMM_MAX_TOKENS and (rows > 8192 or tokens * rows > _SHARED_FUSED_MAX):
         return None
     return ext().fused_affine_gate_up_silu_gemm(x, [_entry(g), _entry(u)])
 

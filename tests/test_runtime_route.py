@@ -150,3 +150,29 @@ def test_decode_sweep_batch_rule(monkeypatch, fmt, H, B, ok):
     lm = {"buffer": _Buf(), "shape": [640, H], "gguf_type": fmt, "offset": 0}
     with pytest.raises(Stop if ok else ValueError):
         scheduler.DecodeSweep([_sweep_layer(fmt, H, 2 * H)], lm, batch=B, device="cpu")
+
+
+# (ffn rows, tokens, fused faster): the shared expert's gate/up/SiLU launch
+# against the separate projections (separate / fused us per chunk, in_dim 4096).
+SHARED_TABLE = [
+    (1024, 9, True),       # 37 / 18
+    (1024, 4096, True),    # 99 / 86
+    (2048, 2048, True),    # 98 / 86
+    (2048, 4096, False),   # 162 / 168
+    (4096, 1024, True),    # 101 / 88
+    (4096, 2048, False),   # 164 / 171
+    (8192, 512, True), (8192, 513, False),
+]
+
+
+@pytest.mark.parametrize("rows,tokens,fused", SHARED_TABLE)
+def test_shared_expert_gate_up_route(monkeypatch, rows, tokens, fused):
+    class Fused:
+        def fused_affine_gate_up_silu_gemm(self, x, entries):
+            return x
+
+    monkeypatch.setattr(qwen_moe, "ext", lambda: Fused())
+    meta = {"buffer": _Buf(), "shape": [rows, 256], "quant_type": "affine_q4", "weight_offset": 0,
+            "scale_offset": 0, "bias_offset": 0, "group_size": 64}
+    weights = {f"mlp.shared_expert.{p}_proj.weight": meta for p in ("gate", "up")}
+    assert (qwen_moe._shared_gate_up_silu(torch.zeros(1, tokens, 256), weights) is not None) == fused
