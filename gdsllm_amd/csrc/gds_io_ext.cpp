@@ -505,12 +505,17 @@ std::optional<torch::Tensor> moe_step_affine_q4(torch::Tensor x, std::vector<Aff
 }
 
 // The partial-sum workspace of a prefill GEMM that splits K, from torch's
-// allocator on the current stream (undefined where the library does not split).
+// allocator on the current stream; undefined where the library does not split
+// and where the memory is not there (the launch then takes K whole).
 torch::Tensor gemm_workspace(int64_t out_dim, int64_t in_dim, int64_t tokens, int dev, bool gate_up = false) {
     const auto bytes = static_cast<int64_t>((gate_up ? gdsllm_dequant_gemm_gate_up_silu_workspace_size
                                                      : gdsllm_dequant_gemm_workspace_size)(out_dim, in_dim, tokens));
     if (bytes == 0) return {};
-    return torch::empty({bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, dev));
+    try {
+        return torch::empty({bytes}, torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA, dev));
+    } catch (const c10::OutOfMemoryError&) {
+        return {};
+    }
 }
 
 // Prefill: x [..., in_dim] fp16 -> [..., out_dim] fp16 on the MFMA dequant-GEMM

@@ -638,3 +638,34 @@ def test_dequant_gemm_gate_up_silu_split_k(gpu, fmt, T, F, K):
     sg = np.abs(oq.silu_fp16(gq).astype(np.float64))
     bound = 2 * ((1.1 * eg + oq.fp16_ulp(sg)) * (np.abs(uq.astype(np.float64)) + eu) + sg * eu + oq.fp16_ulp(want))
     assert (np.abs(a - b) <= bound).all()
+
+
+def test_dequant_gemm_workspace_out_of_memory(gpu):
+    """A chunk whose K-split workspace does not fit in device memory runs with K
+    whole (the bits of the entry without a workspace), as it did before there
+    was one; with memory it splits."""
+    from gdsllm_amd.runtime import ext
+
+    T, M, K = 100, 2048, 11008
+    assert capi().gdsllm_dequant_gemm_workspace_size(M, K, T) > 2 << 20
+    w, x = syn.q8_0_weights(M, K, gen(6001)).reshape(-1).to(gpu), syn.activations(T, K, gen(6002)).to(gpu)
+    handle, whole = ext().GdsBufferHandle.from_tensor(w), torch.empty(T, M, dtype=torch.float16, device=gpu)
+    check(capi().gdsllm_dequant_gemm_q8_0(ptr(w), ptr(x), ptr(whole), M, K, T, K, M, stream()))
+    run = lambda: ext().fused_dequant_gemm(handle, x.view(1, T, K), [M, K], "q8_0", 0)[0]  # noqa: E731
+    split = run()
+    hold = [torch.empty(T, M, dtype=torch.float16, device=gpu)]  # an output's place, freed below
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(gpu).total_memory
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(gpu) / total, gpu)
+    try:
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:  # fill what the cached blocks of this size have left
+                hold.append(torch.empty(2 << 20, dtype=torch.uint8, device=gpu))
+        hold.pop(0)
+        got = run()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, gpu)
+    assert torch.equal(got, whole)
+    a, b = to_np(split).astype(np.float64), to_np(whole).astype(np.float64)
+    assert np.linalg.norm(a - b) <= 2.0 ** -10 * np.linalg.norm(b)
