@@ -669,3 +669,38 @@ def test_dequant_gemm_workspace_out_of_memory(gpu):
     assert torch.equal(got, whole)
     a, b = to_np(split).astype(np.float64), to_np(whole).astype(np.float64)
     assert np.linalg.norm(a - b) <= 2.0 ** -10 * np.linalg.norm(b)
+
+
+def split_plan(gpu, rows, T, K):
+    """(tile tokens, parts) of the K-split rule of prefill.hip's pick_split."""
+    cu, unit = torch.cuda.get_device_properties(gpu).multi_processor_count, 22.0 * K / 4096
+    jobs = lambda bm, bt: -(-rows // bm) * -(-T // bt)  # noqa: E731
+    whole = min(-(-jobs(bm, bt) // cu) * (5 + r * unit) for bm, bt, r in ((128, 64, 1.1), (128, 128, 1.7), (256, 128, 2.6)))
+    plans = [(5 + r * unit / p + 4 + 8 * p * T * rows / 4e6, bt, p) for bt, r in ((128, 1.7), (64, 1.1))
+             for p in range(2, 9) if K // 256 / p >= 4 and jobs(128, bt) * p <= cu]
+    cost, bt, parts = min(plans, key=lambda c: c[0], default=(whole, 0, 1))
+    return (bt, parts) if cost < 0.95 * whole else (0, 1)
+
+
+# Shapes that split with the 128-token tile (two accumulator passes; the cases
+# above take the 64-token one): ragged token tiles, rows off the 128 grid and
+# off the 4-row store.
+WIDE_CASES = [(450, 1290, 4096), (333, 2001, 4096), (450, 1026, 8192)]
+WIDE_DUAL_CASES = [(400, 777, 4096), (450, 777, 5888), (257, 1290, 4096)]
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "affine32", "affine64", "affine128"])
+@pytest.mark.parametrize("T,M,K", WIDE_CASES, ids=[f"T{t}_{m}x{k}" for t, m, k in WIDE_CASES])
+def test_dequant_gemm_split_k_wide_tile(gpu, fmt, T, M, K):
+    bt, parts = split_plan(gpu, M, T, K)
+    assert bt == 128 and capi().gdsllm_dequant_gemm_workspace_size(M, K, T) == parts * T * -(-M // 4) * 16
+    test_dequant_gemm_split_k(gpu, fmt, T, M, K)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "affine32", "affine64", "affine128"])
+@pytest.mark.parametrize("T,F,K", WIDE_DUAL_CASES, ids=[f"T{t}_{m}x{k}" for t, m, k in WIDE_DUAL_CASES])
+def test_dequant_gemm_gate_up_silu_split_k_wide_tile(gpu, fmt, T, F, K):
+    bt, parts = split_plan(gpu, 2 * F, T, K)
+    need = capi().gdsllm_dequant_gemm_gate_up_silu_workspace_size(F, K, T)
+    assert bt == 128 and need == 2 * parts * T * -(-F // 4) * 16
+    test_dequant_gemm_gate_up_silu_split_k(gpu, fmt, T, F, K)
