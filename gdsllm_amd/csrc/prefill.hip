@@ -178,8 +178,10 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 // bounds this kernel at 512 tokens.  A wave's stage is two sub-stages (its two
 // blocks of the four), each scheduled like a 128-row stage; the wait and the
 // workgroup barrier come once per stage, after the second.
-template <WF F, int BT, int MODE, int BM = kBM>
-__global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
+//
+// gemm_job is job b of the launch's `jobs`.
+template <WF F, int BT, int MODE, int BM>
+__device__ __forceinline__ void gemm_job(const GemmArgs& a, int b, int jobs) {
     using Fm = Fmt<F, BM>;
     using R = Ring<F, BT, BM>;
     constexpr int NTF = BT / 32;        // token fragments per wave
@@ -205,13 +207,9 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
     int64_t k0 = 0;  // first k of this workgroup's part (split modes)
     const uint8_t *wA = a.w, *sA = a.s, *bA = a.b, *wB = a.w2, *sB = a.s2, *bB = a.b2;
     if constexpr (kGath) {
-        // The grid covers the worst case; the first ntiles * mtiles
-        // workgroups take a job, in the XCD-aware order of the dense modes
-        // over that count: an XCD takes a contiguous range of jobs, i.e. the
-        // row tiles of the same experts, so an expert's token rows of X come
-        // into one L2, not into all eight.
-        const int jobs = __builtin_amdgcn_readfirstlane(*a.ntiles) * a.mtiles, b = blockIdx.x;
-        if (b >= jobs) return;  // uniform
+        // The XCD-aware order of the dense modes: an XCD takes a contiguous
+        // range of jobs, i.e. the row tiles of the same experts, so an expert's
+        // token rows of X come into one L2, not into all eight.
         const int per = jobs >> 3, rem = jobs & 7, xcd = b & 7;
         const int q = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
         const int tile = q / a.mtiles;
@@ -231,8 +229,7 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
         }
     } else {
         // XCD-aware order: dispatch sends workgroup b to XCD b % 8
-        const int nwg = gridDim.x, b = blockIdx.x;
-        const int per = nwg >> 3, rem = nwg & 7, xcd = b & 7;
+        const int per = jobs >> 3, rem = jobs & 7, xcd = b & 7;
         const int q = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
         m0 = (q % a.mtiles) * (kDual ? BM / 2 : BM);
         int tt = q / a.mtiles;
@@ -712,12 +709,36 @@ __global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
     }
 }
 
-template <WF F, int BT, int MODE, int BM = kBM>
+// LOOP: a workgroup takes jobs blockIdx.x, += gridDim.x of a gathered launch,
+// for grids that may find no job at all (each workgroup of such a grid costs
+// 0.4-0.6 ns: of 8 and 13.5 us, traced, beside the streams of 512 tokens over
+// 512 experts).
+// With a job per workgroup the products themselves are up to 3% faster, so the
+// other launches keep that.
+template <WF F, int BT, int MODE, int BM, bool LOOP>
+__global__ __launch_bounds__(kWaves * 64) void gemm_sk(GemmArgs a) {
+    if constexpr (MODE == kGather || MODE == kDualSilu) {
+        // the grid covers the worst case; the first ntiles * mtiles jobs exist
+        const int jobs = __builtin_amdgcn_readfirstlane(*a.ntiles) * a.mtiles;
+        if constexpr (LOOP) {
+            for (int b = blockIdx.x; b < jobs; b += gridDim.x) {
+                gemm_job<F, BT, MODE, BM>(a, b, jobs);
+                __syncthreads();  // the next job's transfers reuse the LDS
+            }
+        } else {
+            if (static_cast<int>(blockIdx.x) < jobs) gemm_job<F, BT, MODE, BM>(a, blockIdx.x, jobs);  // uniform
+        }
+    } else {
+        gemm_job<F, BT, MODE, BM>(a, blockIdx.x, gridDim.x);
+    }
+}
+
+template <WF F, int BT, int MODE, int BM = kBM, bool LOOP = false>
 int launch_sk(const GemmArgs& a, unsigned nwg, hipStream_t stream) {
     using R = Ring<F, BT, BM>;
-    const void* fn = reinterpret_cast<const void*>(&gemm_sk<F, BT, MODE, BM>);
+    const void* fn = reinterpret_cast<const void*>(&gemm_sk<F, BT, MODE, BM, LOOP>);
     if (int rc = prepare_lds(fn, R::kLds)) return rc;
-    hipLaunchKernelGGL((gemm_sk<F, BT, MODE, BM>), dim3(nwg), dim3(kWaves * 64), R::kLds, stream, a);
+    hipLaunchKernelGGL((gemm_sk<F, BT, MODE, BM, LOOP>), dim3(nwg), dim3(kWaves * 64), R::kLds, stream, a);
     return check_hip(hipGetLastError(), "prefill gemm launch");
 }
 
@@ -1088,7 +1109,7 @@ constexpr int kMoeBT = 32;
 // 895, 1125 / 1064 and 518 / 608.  Where the host knows the answer (even routing
 // at random would leave too few passes, or the mean load is past 16) only the
 // tiles are launched; else the pair of launches that moe_sort leaves empty
-// takes 3 us, up to 11 where the empty tile grid is large.
+// takes about 3 us.
 inline MoePath moe_path(int64_t T, int64_t k, int64_t E, int64_t H, int64_t Fd) {
     const MoePath tiles{INT_MAX, 0, 1};
     if (!moe_stream_fits(Fd, H) || !moe_stream_fits(H, Fd) || T * k > kStreamTokens * E) return tiles;
@@ -1099,14 +1120,17 @@ inline MoePath moe_path(int64_t T, int64_t k, int64_t E, int64_t H, int64_t Fd) 
     return {min_passes, 27, 20};
 }
 
-// Most tiles the split-K launches can get: of n entries over E experts, and
-// where streams are the other choice, fewer than min_passes or a share ntwo /
-// tiles > (num - den) / den of two-pass tiles, of 17 entries or more each.
-inline int64_t max_gemm_tiles(const MoePath& path, int64_t n, int64_t E) {
-    const int64_t all = n / kMoeBT + std::min<int64_t>(E, n);
-    if (path.min_passes == INT_MAX) return all;
-    const int64_t loaded = n * path.den / (path.den + kStreamTokens * (path.num - path.den));
-    return std::min(all, std::max<int64_t>(path.min_passes, loaded));
+// A gathered launch over at most max_jobs tiles: where the streams may have
+// taken the chunk and an empty grid would be large, at most 8 workgroups per
+// compute unit, looping (512 tokens over 512 experts: 1% of the chunk, 861 ->
+// 849 us with Zipf(1) routing; chunks of a few experts, whose grids are small,
+// lost up to a microsecond by it).
+template <WF F, int MODE>
+int gather_gemm(const GemmArgs& a, const MoePath& path, int64_t max_jobs, hipStream_t stream) {
+    const int64_t cu = cu_count();
+    if (path.min_passes == INT_MAX || max_jobs <= 32 * cu)
+        return launch_sk<F, kMoeBT, MODE>(a, static_cast<unsigned>(max_jobs), stream);
+    return launch_sk<F, kMoeBT, MODE, kBM, true>(a, static_cast<unsigned>(8 * cu), stream);
 }
 
 struct PrefillLayout {
@@ -1150,7 +1174,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     hipLaunchKernelGGL(moe_sort, dim3(1), dim3(kSortThreads), 0, stream, idx, static_cast<int>(n), static_cast<int>(k),
                        static_cast<int>(E), kMoeBT, path, tok, pos, tiles, counts);
     if (int rc = check_hip(hipGetLastError(), "moe_sort launch")) return rc;
-    const int64_t max_tiles = max_gemm_tiles(path, n, E);
+    const int64_t max_tiles = n / kMoeBT + std::min<int64_t>(E, n);
     auto combine = [&]() {
         const int64_t threads = T * (H / 8);
         hipLaunchKernelGGL(moe_prefill_combine, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, stream,
@@ -1215,7 +1239,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     a.tiles = tiles;
     a.ntiles = counts + 1;
     a.tok = tok;
-    if (int rc = launch_sk<F, kMoeBT, kDualSilu>(a, static_cast<unsigned>(max_tiles * a.mtiles), stream)) return rc;
+    if (int rc = gather_gemm<F, kDualSilu>(a, path, max_tiles * a.mtiles, stream)) return rc;
 
     GemmArgs b{};
     b.w = static_cast<const uint8_t*>(d.weight);
@@ -1238,7 +1262,7 @@ int moe_prefill_run(const gdsllm_affine_experts& g, const gdsllm_affine_experts&
     b.tiles = tiles;
     b.ntiles = counts + 1;
     b.tok = nullptr;
-    if (int rc = launch_sk<F, kMoeBT, kGather>(b, static_cast<unsigned>(max_tiles * b.mtiles), stream)) return rc;
+    if (int rc = gather_gemm<F, kGather>(b, path, max_tiles * b.mtiles, stream)) return rc;
     return combine();
 }
 

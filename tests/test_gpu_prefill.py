@@ -241,9 +241,9 @@ def test_moe_prefill(gpu, E, H, F, g, k, T):
     assert torch.equal(y.view(torch.int16), y2.view(torch.int16))
 
 
-# (E, H, F, g, k, T) with few tokens per expert, the streamed form: K of 256 and
-# 768 (half-size units), 512 and 1536 (scales of one unit a load), 1024 and 2048
-# (two and four), rows past a job's range (H = 1280), every group size
+# (E, H, F, g, k, T) with few tokens per expert: K of 256 and 768, 512 and 1536,
+# 1024 and 2048, rows past a job's range (H = 1280), every group size (the chunks
+# are too small for the weight streams; test_moe_prefill_paths has those)
 STREAM_CASES = [(40, 1024, 512, 64, 4, 30), (40, 768, 256, 64, 2, 40), (24, 2048, 1024, 128, 3, 20),
                 (24, 1536, 512, 32, 3, 20), (24, 1280, 768, 128, 2, 30), (130, 512, 256, 32, 4, 200),
                 (24, 2048, 256, 32, 2, 9)]
@@ -288,14 +288,15 @@ def _moe_paths(dev, xd, idx_d, wts_d, g, T, k):
 # passes (17, 31, 32, 33 and 48 tokens), one or two jobs per pass, rows past a
 # job's range (H = 1280), K of 256 .. 2048 and every group size; then the same
 # pools with the load on a few experts or too few passes, which the device gives
-# to the split-K tiles; then what the host gives to them by itself: a mean load
+# to the split-K tiles (the last one more tiles than its looping grid has
+# workgroups); then what the host gives to them by itself: a mean load
 # past 16, few experts, a hidden size no stream takes.
 PATH_CASES = [
-    (60, 2048, 1024, 64, 3, 60, (17, 31), True), (180, 256, 256, 32, 4, 80, (32, 33), True),
+    (60, 2048, 1024, 64, 3, 60, (17, 31), True), (60, 2048, 1024, 128, 3, 60, (20,), True), (180, 256, 256, 32, 4, 80, (32, 33), True),
     (80, 1536, 512, 128, 3, 70, (48,), True), (70, 1280, 768, 64, 2, 100, (16, 1), True),
     (150, 768, 256, 64, 3, 120, (), True), (110, 1024, 512, 32, 3, 90, (40,), True),
     (60, 2048, 1024, 64, 3, 60, None, False), (180, 256, 256, 32, 4, 80, None, False),
-    (60, 2048, 1024, 32, 3, 39, "few", False),
+    (60, 2048, 1024, 32, 3, 39, "few", False), (512, 2048, 256, 64, 10, 512, None, False),
     (6, 1024, 256, 32, 3, 40, (), False), (4, 4096, 1024, 64, 2, 70, (33,), False), (60, 4608, 256, 32, 2, 70, (), False),
 ]
 

@@ -135,7 +135,7 @@ def _sweep_layer(fmt, H, F):
                                         ("q4_0", 512, 9, False), ("q4_0", 512, 0, False), ("q5_0", 512, 1, False)])
 def test_decode_sweep_batch_rule(monkeypatch, fmt, H, B, ok):
     """DecodeSweep takes batch 1-8 for both GGUF types (a gate/up/SiLU launch
-    the fused kernel refuses runs as two GEMVs and torch's SiLU and product);
+    the fused kernel refuses runs as a grouped launch and an elementwise one);
     other batches and types are refused before any device memory is
     allocated."""
     from gdsllm_amd.runtime import scheduler
