@@ -53,21 +53,21 @@ def _fused_dequant_gemv(x: torch.Tensor, meta: dict) -> torch.Tensor:
 # Measured on MI355X: the fused MFMA dequant-GEMM against the bit-exact dequant
 # into a scratch matrix + hipBLASLt (the reference's route), Q4_0, Q8_0 and
 # affine-Q4 g64 over 4096x4096, 11008x4096, 4096x11008, 32000x4096, 8192x8192,
-# 1024x8192, 28672x8192, 8192x28672 and 2048x4096 at 64 to 1024 tokens.
-#  * Q4_0 and affine-Q4: the fused GEMM wins wherever its 128-row x 64-token
-#    tiles number at least 32 (64 over an in_dim past 8192, where each tile is
-#    long, or over 2048 rows), on 2048 rows or more, for chunks of up to 512
-#    tokens, and for longer chunks over up to 8192 rows (8192x28672 at 1024
-#    tokens: 464 against 503 us); it loses on 1024 rows (1024x8192 at 512
-#    tokens: 51 against 40 us), where few tiles leave most compute units idle
-#    (4096x11008 at 64 tokens: 62 against 53 us), and at 1024 tokens over
-#    11008 rows or more (11008x4096: 132 against 108 us), where it dequantizes
-#    every weight once per token tile and the route once per call.
-#  * Q8_0 (a W stage twice Q4_0's): the fused GEMM wins on 8192 rows or more
-#    up to 512 tokens (28672x8192 at 128 tokens: 97 against 247 us), except
-#    512 tokens over an in_dim of 4096 on fewer than 16384 rows (11008x4096:
-#    82 against 76 us); on 4096 rows the two are within 10% either way and the
-#    route is taken.
+# 1024x8192, 28672x8192, 8192x28672 and 2048x4096 at 9 to 1024 tokens (us).
+#  * Q4_0 and affine-Q4: the fused GEMM for chunks of up to 512 tokens (28672x8192
+#    at 64: 47 against 230; 11008x4096 at 512: 61 against 69), and for longer
+#    chunks over up to 8192 rows (8192x28672 at 1024: 405 against 476); past them
+#    it dequantizes every weight once per token tile and the route once per
+#    call (11008x4096 at 1024: 119 against 99).
+#  * Q8_0 (a W stage twice Q4_0's): on 8192 rows or more up to 512 tokens
+#    (28672x8192 at 128: 87 against 238), except 512 tokens over an in_dim of 4096 on
+#    fewer than 16384 rows (11008x4096: 74 against 71).
+#  * The lower lines (128-row x 64-token tiles, rows, Q8_0's rows) were drawn from
+#    launches with K whole, where few tiles leave most compute units idle.  With K
+#    split over them the fused GEMM is the faster one below those lines too
+#    (Q4_0 4096x11008 at 64: 20 against 52, 1024x8192 at 128: 16 against 25; Q8_0
+#    4096x4096 at 64: 17 against 27, 4096x11008 at 256: 43 against 66): the rule keeps to
+#    the route there all the same.
 FUSED_GEMM_MAX_TOKENS = 512
 FUSED_GEMM_MIN_ROWS = 2048
 

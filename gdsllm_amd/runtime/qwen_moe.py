@@ -152,7 +152,9 @@ def _shared_gate_up_silu(x: torch.Tensor, weights: Dict) -> Optional[torch.Tenso
     if not all(isinstance(m, dict) and m.get("quant_type") == "affine_q4" and len(m["shape"]) == 2 for m in (g, u)):
         return None
     if list(g["shape"]) != list(u["shape"]) or g["group_size"] != u["group_size"] or \
-            g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8) or not untransformed(x):
+            g["buffer"].device_id != u["buffer"].device_id or (x.shape[1] == 1 and x.shape[0] <= 8):
+        return None
+    if not untransformed(x):
         return None
     tokens, rows = x.numel() // x.shape[-1], 2 * int(g["shape"][0])
     if tokens > FUSED_GEMM_MAX_TOKENS and (rows > 8192 or tokens * rows > _SHARED_FUSED_MAX):

@@ -292,12 +292,14 @@ def _moe_paths(dev, xd, idx_d, wts_d, g, T, k):
 # workgroups); then what the host gives to them by itself: a mean load
 # past 16, few experts, a hidden size no stream takes.
 PATH_CASES = [
-    (60, 2048, 1024, 64, 3, 60, (17, 31), True), (60, 2048, 1024, 128, 3, 60, (20,), True), (180, 256, 256, 32, 4, 80, (32, 33), True),
+    (60, 2048, 1024, 64, 3, 60, (17, 31), True), (60, 2048, 1024, 128, 3, 60, (20,), True),
+    (180, 256, 256, 32, 4, 80, (32, 33), True),
     (80, 1536, 512, 128, 3, 70, (48,), True), (70, 1280, 768, 64, 2, 100, (16, 1), True),
     (150, 768, 256, 64, 3, 120, (), True), (110, 1024, 512, 32, 3, 90, (40,), True),
     (60, 2048, 1024, 64, 3, 60, None, False), (180, 256, 256, 32, 4, 80, None, False),
     (60, 2048, 1024, 32, 3, 39, "few", False), (512, 2048, 256, 64, 10, 512, None, False),
-    (6, 1024, 256, 32, 3, 40, (), False), (4, 4096, 1024, 64, 2, 70, (33,), False), (60, 4608, 256, 32, 2, 70, (), False),
+    (6, 1024, 256, 32, 3, 40, (), False), (4, 4096, 1024, 64, 2, 70, (33,), False),
+    (60, 4608, 256, 32, 2, 70, (), False),
 ]
 
 
@@ -676,7 +678,8 @@ def split_plan(gpu, rows, T, K):
     """(tile tokens, parts) of the K-split rule of prefill.hip's pick_split."""
     cu, unit = torch.cuda.get_device_properties(gpu).multi_processor_count, 22.0 * K / 4096
     jobs = lambda bm, bt: -(-rows // bm) * -(-T // bt)  # noqa: E731
-    whole = min(-(-jobs(bm, bt) // cu) * (5 + r * unit) for bm, bt, r in ((128, 64, 1.1), (128, 128, 1.7), (256, 128, 2.6)))
+    whole = min(-(-jobs(bm, bt) // cu) * (5 + r * unit)
+                for bm, bt, r in ((128, 64, 1.1), (128, 128, 1.7), (256, 128, 2.6)))
     plans = [(5 + r * unit / p + 4 + 8 * p * T * rows / 4e6, bt, p) for bt, r in ((128, 1.7), (64, 1.1))
              for p in range(2, 9) if K // 256 / p >= 4 and jobs(128, bt) * p <= cu]
     cost, bt, parts = min(plans, key=lambda c: c[0], default=(whole, 0, 1))

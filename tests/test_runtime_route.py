@@ -1,6 +1,6 @@
 """The runtime's prefill route choice (CPU): dequant_linear and
 affine_q4_linear take the fused MFMA dequant-GEMM for the chunks where it was
-measured faster than the reference's dequant -> F.linear route
+measured faster, K whole, than the reference's dequant -> F.linear route
 (runtime/llama.py:160-166, runtime/qwen_moe.py:69-73), and that route
 otherwise; a chunk the fused GEMM declines (None) falls back to the route.
 The extension is replaced by a recorder, so no kernel runs."""
@@ -35,33 +35,34 @@ class Recorder:
         return torch.zeros(shape, dtype=torch.float32)
 
 
-# (format, out_dim, in_dim, tokens, fused faster): the choices the route rule
-# must make, each from the MI355X measurement of both routes that the rule in
-# runtime/llama.py summarizes (fused / route us per call in the comments).
+# (format, out_dim, in_dim, tokens, takes the fused GEMM): the choices of the
+# route rule in runtime/llama.py, with fused / route us per call on MI355X.  The
+# rule was drawn from launches with K whole; "split" marks the pairs it leaves to
+# the route though the launch that splits K is the faster one.
 ROUTE_TABLE = [
-    ("q4_0", 4096, 4096, 64, True),        # 29.9 / 34.4
-    ("q4_0", 11008, 4096, 512, True),      # 70.4 / 73.9
-    ("q4_0", 11008, 4096, 1024, False),    # 132.2 / 108.1
-    ("q4_0", 4096, 11008, 64, False),      # 62.5 / 52.8: 32 long tiles
-    ("q4_0", 4096, 11008, 128, True),      # 63.7 / 72.4
-    ("q4_0", 4096, 11008, 1024, True),     # 107.8 / 117.6
-    ("q4_0", 32000, 4096, 1024, False),    # 289.6 / 265.9
-    ("q4_0", 8192, 28672, 1024, True),     # 463.7 / 502.9
-    ("q4_0", 28672, 8192, 64, True),       # 58.1 / 229.3
-    ("q4_0", 1024, 8192, 512, False),      # 50.8 / 40.3
-    ("q4_0", 2048, 4096, 128, False),      # 29.9 / 27.6
-    ("q4_0", 2048, 4096, 512, True),       # 32.7 / 34.8
-    ("q8_0", 11008, 4096, 512, False),     # 82.1 / 76.1
-    ("q8_0", 11008, 4096, 256, True),      # 52.6 / 68.6
-    ("q8_0", 4096, 11008, 256, False),     # 79.7 / 71.7
-    ("q8_0", 4096, 4096, 64, False),       # 34.5 / 31.3
-    ("q8_0", 28672, 8192, 128, True),      # 96.6 / 247.2
-    ("q8_0", 8192, 8192, 512, True),       # 98.4 / 106.3
-    ("q8_0", 8192, 8192, 1024, False),     # 164.4 / 155.6
-    ("q8_0", 32000, 4096, 256, True),      # 89.0 / 150.8
-    ("affine_q4", 4096, 4096, 1024, True),     # 50.9 / 54.4
-    ("affine_q4", 28672, 8192, 1024, False),   # 537.1 / 501.7
-    ("affine_q4", 1024, 8192, 128, False),     # 47.6 / 28.4
+    ("q4_0", 4096, 4096, 64, True),          # 15.8 / 30.4
+    ("q4_0", 11008, 4096, 512, True),        # 60.9 / 68.6
+    ("q4_0", 11008, 4096, 1024, False),      # 118.7 / 99.4
+    ("q4_0", 4096, 11008, 64, False),        # 19.9 / 51.5, split
+    ("q4_0", 4096, 11008, 128, True),        # 26.3 / 69.6
+    ("q4_0", 4096, 11008, 1024, True),       # 99.2 / 109.9
+    ("q4_0", 32000, 4096, 1024, False),      # 276.5 / 245.7
+    ("q4_0", 8192, 28672, 1024, True),       # 405.1 / 475.7
+    ("q4_0", 28672, 8192, 64, True),         # 47.4 / 230.0
+    ("q4_0", 1024, 8192, 512, False),        # 23.4 / 32.0, split
+    ("q4_0", 2048, 4096, 128, False),        # 15.3 / 24.6, split
+    ("q4_0", 2048, 4096, 512, True),         # 22.6 / 29.1
+    ("q8_0", 11008, 4096, 512, False),       # 73.7 / 71.0
+    ("q8_0", 11008, 4096, 256, True),        # 44.7 / 62.5
+    ("q8_0", 4096, 11008, 256, False),       # 43.1 / 65.8, split
+    ("q8_0", 4096, 4096, 64, False),         # 16.8 / 26.9, split
+    ("q8_0", 28672, 8192, 128, True),        # 87.4 / 238.0
+    ("q8_0", 8192, 8192, 512, True),         # 92.9 / 100.7
+    ("q8_0", 8192, 8192, 1024, False),       # 158.5 / 141.8
+    ("q8_0", 32000, 4096, 256, True),        # 83.5 / 143.8
+    ("affine_q4", 4096, 4096, 1024, True),   # 47.9 / 49.3
+    ("affine_q4", 28672, 8192, 1024, False), # 549.5 / 455.8
+    ("affine_q4", 1024, 8192, 128, False),   # 15.9 / 24.1, split
 ]
 
 
@@ -74,7 +75,7 @@ def test_prefill_route_rule(fmt, M, K, T, fused):
     ("q4_0", 11008, 512, True), ("q4_0", 4096, 128, True), ("q4_0", 32000, 512, True), ("q4_0", 28672, 64, True),
     ("q4_0", 11008, 1024, False), ("q4_0", 32000, 2048, False),   # long chunks: dequant once, then the library GEMM
     ("q4_0", 1024, 512, False), ("q4_0", 1024, 64, False),        # short matrices
-    ("q4_0", 2048, 64, False),                                    # 16 tiles: most compute units idle
+    ("q4_0", 2048, 64, False),                                    # 16 tiles
     ("q8_0", 11008, 512, False), ("q8_0", 11008, 256, True), ("q8_0", 4096, 128, False),
 ])
 def test_gguf_prefill_route(monkeypatch, fmt, M, T, fused):
