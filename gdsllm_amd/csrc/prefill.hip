@@ -838,8 +838,13 @@ __global__ __launch_bounds__(256) void split_sum(const float* __restrict__ part,
 // (128, 4); 11008 x 4096 at 60 33.5 -> 24.5 (64, 2); Q4_0 4096 x 11008 at 128 /
 // 256 / 333 56.7 -> 27.2 (64, 4) / 57.8 -> 38.7 (128, 4) / 59.1 -> 55.1 (128,
 // 2); 4096 x 4096 at 64 24.9 -> 15.5 (64, 4); 2048 x 4096 at 512 25.4 -> 23.1
-// (64, 2).  4096 x 11008 at 512 (64.6 -> 61.9, 128 tokens, 2 parts) stays whole,
-// and so does every launch of over half a round of tiles.
+// (64, 2); affine 4096 x 4096 at 64 24.4 -> 15.5, 4096 x 11008 at 256 59.4 ->
+// 39.8, gate/up of 1024 x 4096 at 9 / 512 24.2 -> 14.0 / 26.1 -> 23.7.  4096 x
+// 11008 at 512 (64.6 -> 61.9, 128 tokens, 2 parts) stays whole, and so does
+// every launch of over half a round of tiles.  The whole-launch estimate here
+// and pick_tile's differ in their constants; over the 624 launches that split
+// among 16 matrices, three formats, both modes and 1-512 tokens, 0.27-1.01 of
+// the whole launch's time.
 struct SplitPlan {
     int bt = 0, parts = 1;
 };
