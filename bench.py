@@ -881,7 +881,7 @@ def bench_moe_prefill(dev, tokens: int = 512, reps: int = 5, reference: bool = T
     flops = 2 * tokens * k * 3 * Fd * H
     res = {"us_per_chunk": round(ms * 1e3, 1), "tokens": tokens, "top_k": k, "experts_used": len(used),
            "weight_bytes": wbytes, "weight_GB_s": round(wbytes / (ms * 1e-3) / 1e9, 1),
-           "TFLOP_s": round(flops / (ms * 1e-3) / 1e12, 1), "launches": 4, "host_syncs": 0}
+           "TFLOP_s": round(flops / (ms * 1e-3) / 1e12, 1), "launches": 6, "host_syncs": 0}
     if not reference:
         return res
 

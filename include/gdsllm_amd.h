@@ -399,9 +399,11 @@ size_t gdsllm_moe_prefill_workspace_size(int64_t tokens, int64_t top_k, int64_t 
  *   y[t] = sum over j in order of fp16(w[t][j] * down_e(h)), each product and
  *          partial sum rounded to fp16, e = idx[t][j],
  *   h    = fp16(fp16(silu(fp16(gate_e . x_t))) * fp16(up_e . x_t)).
- * Four launches and no host sync: the entries sorted by expert, one grouped
- * MFMA GEMM for gate/up/SiLU over each expert's tokens, one for down, the
- * combine.  Expert indices outside [0, num_experts) contribute nothing.  No
+ * No host sync: the entries sorted by expert, one grouped MFMA GEMM for
+ * gate/up/SiLU over each expert's tokens, one for down, the combine.  Four
+ * launches, or six where the device settles from the experts' loads which of two
+ * forms of the GEMMs runs (the other finds no work; the forms differ by fp32
+ * reassociation).  Expert indices outside [0, num_experts) contribute nothing.  No
  * counterpart kernel in the reference, which loops over the unique experts
  * with dequant -> F.linear per projection.  Needs hidden and ffn multiples of
  * 256, group_size 32, 64 or 128, gate and up with equal strides, at most 4096
